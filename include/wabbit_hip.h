@@ -524,10 +524,10 @@ int wh_set_tables_from_forests(wh_pool *pool, wh_forest *const *forests, int n, 
  * 0 selects the flat one-point-per-thread kernel, -1 automatic.
  * WH_TUNE_K3D_ZSPLIT (default 1): the z range of a block is cut into zsplit
  * pieces marched by separate workgroups (a split that does not divide Bs2
- * into pieces of at least 2R planes, R the stencil reach, acts as 1).
- * WH_TUNE_K3D_WAVES (default 1): 3 selects the build of the z-marching
- * kernel whose register allocation allows 3 waves per SIMD, 4 the build of
- * the flat kernel allowing 4 (both may spill a few registers).
+ * into pieces of at least 2R planes, R the stencil reach, acts as 1; with the
+ * automatic y-split 1 leaves the z-split to the library too).
+ * WH_TUNE_K3D_WAVES (default 1): 1, 3 or 4, without effect (there is one
+ * build of each 3D kernel, whose registers allow 3 to 5 waves per SIMD).
  * WH_TUNE_K3D_XCD (default 0): 1 remaps the flat 3D kernel's workgroups so
  * that those of one block run on one XCD (one L2).
  * WH_TUNE_K2D_STAGE: 2D stage kernel variant: 0 one workgroup per block;
@@ -541,7 +541,11 @@ int wh_set_tables_from_forests(wh_pool *pool, wh_forest *const *forests, int n, 
  * of every active block, the fused RK stages read each block's halo tile
  * straight from its neighbours' interiors and the step launches no ghost
  * fill (the values are the same copies; the state's own ghost nodes are
- * then not refreshed by the step); 0 fills the ghost nodes first. */
+ * then not refreshed by the step).  In a 3D pool whose stages run the
+ * z-marching kernel the state's ghost nodes are filled as always, and the
+ * later stages read every face that is one whole same-level copy from the
+ * neighbour's interior, so that only the remaining patches are launched on
+ * the stage inputs in the work slots.  0 fills the ghost nodes first. */
 enum {
     WH_TUNE_K3D_YSPLIT = 1,
     WH_TUNE_K2D_STAGE = 2,
@@ -557,7 +561,8 @@ int wh_get_tuning(wh_pool *pool, int key, int *value);
  * pool's (Bs, g, neq) and parameters on the current active blocks, keeps the
  * fastest and returns it (3D: the WH_TUNE_K3D_YSPLIT value, with the
  * WH_TUNE_K3D_ZSPLIT, WH_TUNE_K3D_WAVES and WH_TUNE_K3D_XCD values set as
- * well; 2D: the
+ * well, each variant timed with the ghost fill of a stage input that it
+ * needs; 2D: the
  * WH_TUNE_K2D_STAGE value).  With three or more work slots the timed kernel
  * is the fused RK stage kernel and work slots 0 and 1 are overwritten,
  * otherwise the RHS kernel and work slot 1. */

@@ -116,10 +116,184 @@ static const int32_t *gather_table(wh_pool *P, const AcmDev &a)
     return P->gather_all ? ps.d_gnb : nullptr;
 }
 
+// grow a device buffer to at least n elements (contents are not kept);
+// callers synchronise the stream first
+template <class T>
+static int grow_dev(T *&ptr, size_t &cap, size_t n)
+{
+    if (n <= cap) return WH_OK;
+    if (ptr) WH_HIP(hipFree(ptr));
+    ptr = nullptr;
+    const size_t c = std::max(n, 2 * cap);
+    cap = 0;
+    WH_HIP(hipMalloc(&ptr, sizeof(T) * c));
+    cap = c;
+    return WH_OK;
+}
+
+// host -> pinned staging -> device buffer `dst` (one host-to-device copy),
+// ordered on the pool stream; the pinned space is reused only after a stream
+// synchronisation
+static int upload_staged(wh_pool *P, void *dst, const void *src, size_t bytes)
+{
+    if (!bytes) return WH_OK;
+    if (int rc = stage_begin(P, bytes)) return rc;
+    void *h = stage_host(P, src, bytes);
+    if (!h) return WH_E_HIP;
+    WH_HIP(hipMemcpyAsync(dst, h, bytes, hipMemcpyHostToDevice, P->stream));
+    return WH_OK;
+}
+
+// Does the patch read the sender outside its interior [g, g + Bs)?
+static bool reads_ghosts(const wh_pool *P, const wh_patch &q)
+{
+    for (int d = 0; d < P->d.dim; ++d) {
+        int lo = q.send_lo[d], hi = lo + (q.op == WH_PATCH_RESTRICT ? 2 : 1) * (q.n[d] - 1);
+        if (q.op == WH_PATCH_PREDICT) {
+            const int N = q.aux / 2, f0 = lo, f1 = hi;
+            lo = f0 & 1 ? (f0 >> 1) - N + 1 : f0 < f1 ? std::min(f0 >> 1, ((f0 + 1) >> 1) - N + 1) : f0 >> 1;
+            hi = f1 & 1 ? (f1 >> 1) + N : f0 < f1 ? std::max(f1 >> 1, ((f1 - 1) >> 1) + N) : f1 >> 1;
+        }
+        if (lo < P->d.g || hi >= P->d.g + P->d.bs[d]) return true;
+    }
+    return false;
+}
+
+// The face table of the active blocks (FaceGather) for stencils of reach R.
+// A face is gathered where its R ghost layers (the stencils run along the
+// axes, so edges and corners do not count) are filled by exactly one patch,
+// a first-stage copy of the whole face from the interior of a block one
+// block away, and nothing else writes there: the gather then reads the
+// values that copy would have written.  Of the other first-stage patches
+// those are kept that fill a face that is not gathered, and all those of
+// blocks whose ghost nodes a later patch (restriction, prediction) reads;
+// later stages are kept whole.  A table with a first-stage patch that reads
+// ghost nodes itself is left alone.
+static int build_faces(wh_pool *P, int R)
+{
+    WH_PROF("build_faces");
+    FaceGather &F = P->faces;
+    const PatchSet &ps = P->ps[0];
+    const int dim = P->d.dim, nf = 2 * dim, g = P->d.g;
+    F.any = false;
+    F.h_kept.clear();
+    F.h_chunks.clear();
+    F.h_face.assign((size_t)P->nact * nf, -1);
+    std::vector<int32_t> pos(P->d.nb_max, -1);
+    for (int k = 0; k < P->nact; ++k) pos[P->h_active[k]] = k;
+    std::vector<char> need(P->d.nb_max, 0), closed((size_t)P->nact * nf, 0);
+    // bit f: the patch writes ghost layers of face f that the stencils read
+    auto faces_of = [&](const wh_patch &q) {
+        int in = 0, lo = 0, hi = 0;  // per direction: touches the interior range, the layers below, above
+        for (int d = 0; d < dim; ++d) {
+            const int a = q.recv_lo[d], b = a + q.n[d], e = g + P->d.bs[d];
+            if (a < e && b > g) in |= 1 << d;
+            if (a < g && b > g - R) lo |= 1 << d;
+            if (a < e + R && b > e) hi |= 1 << d;
+        }
+        int m = 0;
+        for (int d = 0; d < dim; ++d)
+            if (((in | 1 << d) == (1 << dim) - 1)) m |= (lo >> d & 1) << (2 * d) | (hi >> d & 1) << (2 * d + 1);
+        return m;
+    };
+    bool ok = true;
+    std::vector<uint8_t> touch(ps.n, 0);
+    for (int i = 0; i < ps.n && ok; ++i) {
+        const wh_patch &q = ps.host[i];
+        if (reads_ghosts(P, q)) {
+            if (q.stage == 1) ok = false;
+            need[q.send] = 1;
+        }
+        const int k = pos[q.recv];
+        if (k < 0) continue;
+        const int m = faces_of(q);
+        touch[i] = (uint8_t)m;
+        for (int f = 0; f < nf; ++f) {
+            if (!(m >> f & 1)) continue;
+            int32_t &at = F.h_face[(size_t)k * nf + f];
+            bool whole = q.op == WH_PATCH_COPY && q.stage == 1 && at < 0;
+            for (int d = 0; d < dim && whole; ++d) {
+                const int a = q.recv_lo[d], b = a + q.n[d], e = g + P->d.bs[d];
+                const int s = d == f >> 1 ? (f & 1 ? -P->d.bs[d] : P->d.bs[d]) : 0;
+                whole = q.send_lo[d] == a + s &&
+                        (d != f >> 1 ? a <= g && b >= e : f & 1 ? a <= e && b >= e + R : a <= g - R && b >= g);
+            }
+            if (whole) at = q.send;
+            else closed[(size_t)k * nf + f] = 1;
+        }
+    }
+    if (ok) {
+        for (size_t i = 0; i < F.h_face.size(); ++i) {
+            if (closed[i]) F.h_face[i] = -1;
+            if (F.h_face[i] >= 0) F.any = true;
+        }
+    }
+    F.reach = R;
+    if (!F.any) return WH_OK;
+    for (int s = 1; s <= 3; ++s) {
+        F.stage_begin[s] = (int)F.h_kept.size();
+        F.chunk_begin[s] = (int)F.h_chunks.size();
+        for (int i = ps.stage_begin[s]; i < ps.stage_begin[s + 1]; ++i) {
+            const wh_patch &q = ps.host[i];
+            bool keep = s > 1 || pos[q.recv] < 0 || need[q.recv];
+            for (int f = 0; f < nf && !keep; ++f)
+                keep = (touch[i] >> f & 1) && F.h_face[(size_t)pos[q.recv] * nf + f] < 0;
+            if (!keep) continue;
+            if (dim == 3) add_chunks(F.h_chunks, (int)F.h_kept.size(), q);
+            F.h_kept.push_back(q);
+        }
+    }
+    F.stage_begin[4] = (int)F.h_kept.size();
+    F.chunk_begin[4] = (int)F.h_chunks.size();
+    if (F.h_face.size() > F.cap_face || F.h_kept.size() > F.cap_kept || F.h_chunks.size() > F.cap_chunks)
+        WH_HIP(hipStreamSynchronize(P->stream));  // before freeing buffers queued work may read
+    if (int rc = grow_dev(F.d_face, F.cap_face, F.h_face.size())) return rc;
+    if (int rc = grow_dev(F.d_kept, F.cap_kept, F.h_kept.size())) return rc;
+    if (int rc = grow_dev(F.d_chunks, F.cap_chunks, F.h_chunks.size())) return rc;
+    if (int rc = upload_staged(P, F.d_face, F.h_face.data(), sizeof(int32_t) * F.h_face.size())) return rc;
+    if (int rc = upload_staged(P, F.d_kept, F.h_kept.data(), sizeof(wh_patch) * F.h_kept.size())) return rc;
+    return upload_staged(P, F.d_chunks, F.h_chunks.data(), sizeof(SyncChunk) * F.h_chunks.size());
+}
+
+// Brings the face table up to date for the fused stages of this scheme (a
+// host-to-device copy where it changed, so before any stream capture).
+static int update_faces(wh_pool *P, const AcmDev &a)
+{
+    if (!P->gather || !stage_gathers(P, a.scheme) || P->nact == 0 || P->ps[0].n == 0) return WH_OK;
+    FaceGather &F = P->faces;
+    const int R = reach_of(a.scheme);
+    if (F.topo == P->topo_version && F.reach == R) return WH_OK;
+    if (F.topo == P->topo_version) P->topo_version++;  // captured graphs hold the other reach's table
+    if (int rc = build_faces(P, R)) return rc;
+    F.topo = P->topo_version;
+    return WH_OK;
+}
+
+// the up-to-date face table, or null where the stages read ghost nodes only
+static const FaceGather *face_table(const wh_pool *P, const AcmDev &a)
+{
+    const FaceGather &F = P->faces;
+    const bool on = P->gather && stage_gathers(P, a.scheme) && F.any && F.topo == P->topo_version &&
+                    F.reach == reach_of(a.scheme);
+    return on ? &F : nullptr;
+}
+
+// the ghost fill that stages with a face table still need
+static int sync_kept(wh_pool *P, const FaceGather &F, double *arr)
+{
+    for (int s = 1; s <= 3; ++s)
+        if (int rc = launch_sync_flat(P, arr, F.d_kept, F.d_chunks, F.stage_begin[s], F.stage_begin[s + 1],
+                                      F.chunk_begin[s], F.chunk_begin[s + 1], SyncSrc{}))
+            return rc;
+    return WH_OK;
+}
+
 // one step of the fused path; dt is taken from the device scalar DS_DT, or
-// per block from dtb (block groups).  With a halo-gather table no ghost
+// per block from dtb (block groups).  With the 2D halo-gather table no ghost
 // fill is launched: every stage reads its blocks' halos from the
-// neighbours' interiors of its input array.
+// neighbours' interiors of its input array.  With a 3D face table the state
+// gets its ghost fill as without it (its ghost nodes are the caller's); of
+// the fills of the stage inputs in the work slots only the kept patches run.
 static int fused_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
                       const double *dtb = nullptr)
 {
@@ -129,13 +303,16 @@ static int fused_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
     double *T[2] = {array_ptr(P, WH_WORK + 1, nullptr, nullptr),
                     array_ptr(P, WH_WORK + 2, nullptr, nullptr)};
     const int32_t *gnb = gather_table(P, a);
+    const FaceGather *fg = face_table(P, a);
     // the ghost fill (timed as a sync launch); nothing at all with gather
     auto sync = [&](double *arr) {
-        return gnb ? (int)WH_OK : timed(P, 1, [&] { return wh::launch_sync(P, 0, arr, -1); });
+        if (gnb || (fg && arr != S && fg->h_kept.empty())) return (int)WH_OK;
+        return timed(P, 1, [&] { return fg && arr != S ? sync_kept(P, *fg, arr) : wh::launch_sync(P, 0, arr, -1); });
     };
     auto launch_fused_stage = [&](wh_pool *Q, const AcmDev &aa, const double *tin, double *tout, const double *u0,
                                   double *ac, double *sout, int mode, double acoef, double bcoef, const double *db) {
-        return wh::launch_fused_stage(Q, aa, tin, tout, u0, ac, sout, mode, acoef, bcoef, db, gnb);
+        return wh::launch_fused_stage(Q, aa, tin, tout, u0, ac, sout, mode, acoef, bcoef, db,
+                                      gnb ? gnb : fg && tin != S ? fg->d_face : nullptr);
     };
     int rc;
     if ((rc = sync(S))) return rc;
@@ -272,21 +449,6 @@ static int check_acm(const wh_pool *P, const wh_acm_params *p)
     return WH_OK;
 }
 
-// grow a device buffer to at least n elements (contents are not kept);
-// callers synchronise the stream first
-template <class T>
-static int grow_dev(T *&ptr, size_t &cap, size_t n)
-{
-    if (n <= cap) return WH_OK;
-    if (ptr) WH_HIP(hipFree(ptr));
-    ptr = nullptr;
-    const size_t c = std::max(n, 2 * cap);
-    cap = 0;
-    WH_HIP(hipMalloc(&ptr, sizeof(T) * c));
-    cap = c;
-    return WH_OK;
-}
-
 static void free_patchset(PatchSet &ps)
 {
     if (ps.d_patches) (void)hipFree(ps.d_patches);
@@ -326,19 +488,6 @@ struct TablesUse {
 static int wait_tables(wh_pool *P)
 {
     if (P->tables_recorded) WH_HIP(hipEventSynchronize(P->ev_tables));
-    return WH_OK;
-}
-
-// host -> pinned staging -> device buffer `dst` (one host-to-device copy),
-// ordered on the pool stream; the pinned space is reused only after a stream
-// synchronisation
-static int upload_staged(wh_pool *P, void *dst, const void *src, size_t bytes)
-{
-    if (!bytes) return WH_OK;
-    if (int rc = stage_begin(P, bytes)) return rc;
-    void *h = stage_host(P, src, bytes);
-    if (!h) return WH_E_HIP;
-    WH_HIP(hipMemcpyAsync(dst, h, bytes, hipMemcpyHostToDevice, P->stream));
     return WH_OK;
 }
 
@@ -431,6 +580,9 @@ int wh_pool_destroy(wh_pool *P)
     destroy_graph(P);
     free_patchset(P->ps[0]);
     free_patchset(P->ps[1]);
+    if (P->faces.d_face) (void)hipFree(P->faces.d_face);
+    if (P->faces.d_kept) (void)hipFree(P->faces.d_kept);
+    if (P->faces.d_chunks) (void)hipFree(P->faces.d_chunks);
     wh::free_wavelet_ws(P);
     for (double *p : {P->block, P->work, P->tmp, P->mask, P->scal, P->d_x0dx})
         if (p) (void)hipFree(p);
@@ -781,7 +933,8 @@ int wh_rk_step(wh_pool *P, const wh_acm_params *p, const double *bt, int nrows, 
     if (path == 2) {
         WH_CHECK(fused_ok(bt, nrows), WH_E_ARG, "tableau not supported by the fused path");
         WH_CHECK(P->d.n_work_slots >= 3, WH_E_ARG, "fused path needs 3 work slots");
-        int rc = launch_set_scalar(P, DS_DT, dt);
+        int rc = update_faces(P, a);
+        if (!rc) rc = launch_set_scalar(P, DS_DT, dt);
         if (rc) return rc;
         return fused_step(P, a, bt, nrows);
     }
@@ -856,6 +1009,7 @@ int wh_rk_step_groups(wh_pool *P, const wh_acm_params *p, const double *bt, int 
     if (path == 2) {
         WH_CHECK(fused_ok(bt, nrows), WH_E_ARG, "tableau not supported by the fused path");
         WH_CHECK(P->d.n_work_slots >= 3, WH_E_ARG, "fused path needs 3 work slots");
+        if (int rc = update_faces(P, a)) return rc;
         if (int rc = upload_staged(P, P->d_dtb, dt_pos.data(), sizeof(double) * P->nact)) return rc;
         return fused_step(P, a, bt, nrows, P->d_dtb);
     }
@@ -929,6 +1083,7 @@ int wh_run_steps(wh_pool *P, const wh_acm_params *p, const double *bt, int nrows
     WH_CHECK(nsteps >= 0, WH_E_ARG, "negative step count");
     const AcmDev a = make_acm_dev(p);
     const TimeDev tc = make_time_dev(tp);
+    if (int rc = update_faces(P, a)) return rc;
     if (!use_graph) {
         for (int s = 0; s < nsteps; ++s) {
             int rc = one_device_step(P, a, bt, nrows, tc);
@@ -1066,13 +1221,16 @@ int wh_time_stage_kernel(wh_pool *P, const wh_acm_params *p, int reps, double *m
     // state and writing only work slots; with the halo-gather table the
     // steps use, the launches gather their halos the same way
     const int32_t *gnb = gather_table(P, a);
+    if (int rc = update_faces(P, a)) return rc;
+    const FaceGather *fg = face_table(P, a);
     auto rk4 = [&]() -> int {
         const double ca[4] = {0.5, 0.5, 1.0, 0.0}, cb[4] = {1.0 / 6.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0};
         const int mode[4] = {0, 1, 1, 2};
         for (int j = 0; j < 4; ++j)
             if (int rc = launch_fused_stage(P, a, P->block, mode[j] == 2 ? nullptr : tout,
                                             mode[j] == 1 ? P->block : nullptr, acc, mode[j] == 2 ? sout : nullptr,
-                                            mode[j], ca[j], cb[j], nullptr, gnb))
+                                            mode[j], ca[j], cb[j], nullptr,
+                                            gnb ? gnb : fg && j > 0 ? fg->d_face : nullptr))
                 return rc;
         return WH_OK;
     };
@@ -1106,25 +1264,33 @@ int wh_autotune(wh_pool *P, const wh_acm_params *p, int reps, int *best_value, d
     std::vector<Var> cand;
     const bool three = P->d.dim == 3;
     if (three) {
-        for (int xcd : {0, 1})
-            for (int wv : {1, 4}) cand.push_back({0, 1, wv, xcd});
+        for (int xcd : {0, 1}) cand.push_back({0, 1, 1, xcd});
         for (int ys = 1; ys <= 8; ++ys)
             for (int zs = 1; zs <= 8; ++zs)
                 if (zm_valid(P->d.bs[0], P->d.bs[1], p->scheme, ys) && zm_zvalid(P->d.bs[2], p->scheme, zs))
-                    for (int wv : {1, 3}) cand.push_back({ys, zs, wv, 0});
+                    cand.push_back({ys, zs, 1, 0});
     } else {
         for (int v = 0; v <= 4; ++v) cand.push_back({v, 1, 1, 0});
     }
     int &knob = three ? P->k3d_ysplit : P->k2d_stage;
     const AcmDev a = make_acm_dev(p);
     double *out = array_ptr(P, WH_WORK + 1, nullptr, nullptr);
-    // with three work slots the timed kernel is the fused RK stage (a middle
+    // with three work slots the timed work is the fused RK stage (a middle
     // stage: reads the block array, the accumulator in work slot 0, writes
-    // work slots 0 and 1), otherwise the RHS; nothing else is written
+    // work slots 0 and 1), in 3D after the ghost fill that the variant needs
+    // (into work slot 1); otherwise the RHS; nothing else is written
     const bool fused = P->d.n_work_slots >= 3;
     double *acc = array_ptr(P, WH_WORK + 0, nullptr, nullptr);
     auto launch = [&]() -> int {
-        if (fused) return launch_fused_stage(P, a, P->block, out, P->block, acc, nullptr, 1, 0.5, 1.0 / 3.0, nullptr);
+        const int32_t *faces = nullptr;
+        if (fused && three) {
+            if (int rc = update_faces(P, a)) return rc;
+            const FaceGather *fg = face_table(P, a);
+            if (int rc = fg ? sync_kept(P, *fg, out) : launch_sync(P, 0, out, -1)) return rc;
+            faces = fg ? fg->d_face : nullptr;
+        }
+        if (fused)
+            return launch_fused_stage(P, a, P->block, out, P->block, acc, nullptr, 1, 0.5, 1.0 / 3.0, nullptr, faces);
         return launch_rhs(P, a, P->block, out, P->d_active, P->d_x0dx, P->nact);
     };
     const Var saved{knob, P->k3d_zsplit, P->k3d_waves, P->k3d_xcd};

@@ -174,6 +174,24 @@ struct PatchSet {
     size_t cap_patches = 0, cap_recv_off = 0, cap_recv_ids = 0, cap_chunks = 0;
 };
 
+// Which faces of the active blocks a fused stage can read straight from the
+// same-level neighbour's interior instead of from ghost nodes, and the RHS
+// ghost patches that are still needed then (wh_api.hip, build_faces).
+struct FaceGather {
+    uint64_t topo = ~0ull;  // topology version and stencil reach it was built for
+    int reach = 0;
+    bool any = false;       // at least one face is gathered
+    std::vector<int32_t> h_face;  // 2*dim ids per active position: -x, +x, -y, +y (, -z, +z); -1: own ghost nodes
+    int32_t *d_face = nullptr;
+    size_t cap_face = 0;
+    std::vector<wh_patch> h_kept;  // patches still launched, by stage
+    std::vector<SyncChunk> h_chunks;
+    wh_patch *d_kept = nullptr;
+    SyncChunk *d_chunks = nullptr;
+    size_t cap_kept = 0, cap_chunks = 0;
+    int stage_begin[5] = {0, 0, 0, 0, 0}, chunk_begin[5] = {0, 0, 0, 0, 0};
+};
+
 }  // namespace wh
 
 struct wh_pool {
@@ -195,6 +213,7 @@ struct wh_pool {
     std::vector<double> h_x0dx;
     int nact = 0, act_cap = 0;
     wh::PatchSet ps[2];
+    wh::FaceGather faces;
     hipStream_t stream = nullptr;
     // timing
     bool timing = false;
@@ -216,7 +235,7 @@ struct wh_pool {
     // tuning: y-split of the 3D stage kernel (-1 auto, 0 flat kernel)
     int k3d_ysplit = -1;
     int k3d_zsplit = 1;
-    int k3d_waves = 1;  // 3: the z-marching kernel built for 3 waves per SIMD, 4: the flat one for 4
+    int k3d_waves = 1;  // WH_TUNE_K3D_WAVES as set (no effect)
     int k3d_xcd = 0;    // 1: the flat 3D kernel's workgroups swizzled per XCD
     // tuning of the 2D stage kernel: 0 plain, 1 mask and epilogue operands
     // loaded before the tile barrier, 2..4 persistent pipelined kernel with
@@ -258,12 +277,15 @@ int launch_combine(wh_pool *P, double *out, const double *base, int nterms,
 int launch_dt(wh_pool *P, const AcmDev &a);
 int launch_maxabs(wh_pool *P, const double *in);
 // dtb: per active-list position dt (block groups), or null for the pool's DS_DT
-// gnb: the halo-gather table of a 2D pool (the ghost fill skipped), or null
+// gnb: 2D: the halo-gather table (the ghost fill skipped), 3D: the face table
+// (FaceGather) of the z-marching kernel, or null
 int launch_fused_stage(wh_pool *P, const AcmDev &a, const double *tin, double *tout,
                        const double *u0, double *acc, double *sout, int mode, double acoef,
                        double bcoef, const double *dtb, const int32_t *gnb = nullptr);
 // per-group minimum block dt into P->d_dtg (bit patterns) for the P->ngrp groups
 int launch_dt_groups(wh_pool *P, const AcmDev &a);
+// whether the 3D stages run the z-marching kernel (the one that can gather)
+bool stage_gathers(const wh_pool *P, int scheme);
 int launch_dt_finalize(wh_pool *P, const TimeDev &tc);
 int launch_time_advance(wh_pool *P);
 int launch_set_scalar(wh_pool *P, int which, double v);

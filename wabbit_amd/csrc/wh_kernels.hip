@@ -83,11 +83,20 @@ __device__ __forceinline__ double d2(const F &f, double inv2)
     }
 }
 
+// a value that is the same in every lane, moved to scalar registers
+__device__ __forceinline__ double wave_uniform(double v)
+{
+    union { double d; int i[2]; } x{v};
+    x.i[0] = __builtin_amdgcn_readfirstlane(x.i[0]);
+    x.i[1] = __builtin_amdgcn_readfirstlane(x.i[1]);
+    return x.d;
+}
+
 // ACM right-hand side at one point (RHS_2D_acm / RHS_3D_acm).  A(c, d, o) is
 // component c of the state at offset o along direction d from the point.
 // mk: mask component 0 at this point (components mcs apart) or null.
 template <int DIM, int S, bool SKEW, class ACC>
-__device__ __forceinline__ void acm_point(const ACC &A, const double *inv, const double *inv2,
+__device__ __forceinline__ void acm_point_all(const ACC &A, const double *inv, const double *inv2,
                                           const AcmDev &a, const double *__restrict__ mk,
                                           ptrdiff_t mcs, double *r)
 {
@@ -144,6 +153,69 @@ __device__ __forceinline__ void acm_point(const ACC &A, const double *inv, const
     }
 }
 
+// The same values with the components one after the other, so that few
+// derivatives are live at once (3D FD4: 90 instead of 144 registers in the
+// flat kernel, 147 instead of 201 in the z-marching one).
+template <int DIM, int S, bool SKEW, class ACC>
+__device__ __forceinline__ void acm_point_seq(const ACC &A, const double *inv, const double *inv2,
+                                          const AcmDev &a, const double *__restrict__ mk,
+                                          ptrdiff_t mcs, double *r)
+{
+    double chi = 0.0, spo = 0.0;
+    if (a.penal && mk) {
+        const int color = (int)mk[4 * mcs];
+        chi = mk[0] * (color == 0 ? 0.0 : a.Cinv);
+    }
+    if (a.sponge && mk) spo = mk[5 * mcs] * a.Csp_inv;
+    double div = 0.0;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+        const double uc = A(c, 0, 0);
+        double du[DIM];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) du[d] = d1<S>([&](int o) { return A(c, d, o); }, inv[d]);
+        double lap = d2<S>([&](int o) { return A(c, 0, o); }, inv2[0]);
+#pragma unroll
+        for (int d = 1; d < DIM; ++d)
+            lap = lap + d2<S>([&](int o) { return A(c, d, o); }, inv2[d]);
+        double t;
+        if constexpr (SKEW) {
+            double sum = d1p<S>([&](int o) { return A(c, 0, o); },
+                                [&](int o) { return A(0, 0, o); }, inv[0]);
+#pragma unroll
+            for (int d = 1; d < DIM; ++d)
+                sum = sum + d1p<S>([&](int o) { return A(c, d, o); },
+                                   [&](int o) { return A(d, d, o); }, inv[d]);
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) sum = sum + A(d, 0, 0) * du[d];
+            t = -(0.5 * sum);
+        } else {
+            t = -(A(0, 0, 0) * du[0]);
+#pragma unroll
+            for (int d = 1; d < DIM; ++d) t = t - A(d, 0, 0) * du[d];
+        }
+        t = t - d1<S>([&](int o) { return A(DIM, c, o); }, inv[c]);
+        t = t + a.nu * lap;
+        if (a.penal && mk) t = t + (-(chi * (uc - mk[(1 + c) * mcs])));
+        if (a.sponge && mk) t = t - (uc - a.ums[c]) * spo;
+        r[c] = t;
+        div = c == 0 ? du[0] : div + du[c];
+    }
+    const double p = A(DIM, 0, 0);
+    r[DIM] = -(a.c02 * div) - a.gamma_p * p;
+    if (a.sponge && mk) r[DIM] = r[DIM] - p * spo;
+}
+
+// 2D: all derivatives first (registers are no limit there, and the loads
+// are all requested at once); 3D: component by component
+template <int DIM, int S, bool SKEW, class ACC>
+__device__ __forceinline__ void acm_point(const ACC &A, const double *inv, const double *inv2, const AcmDev &a,
+                                          const double *__restrict__ mk, ptrdiff_t mcs, double *r)
+{
+    if constexpr (DIM == 2) acm_point_all<DIM, S, SKEW>(A, inv, inv2, a, mk, mcs, r);
+    else acm_point_seq<DIM, S, SKEW>(A, inv, inv2, a, mk, mcs, r);
+}
+
 // accessor over one strided storage: base = component 0 of the point,
 // components cs apart, strides s[d] along direction d
 template <int DIM>
@@ -175,7 +247,9 @@ struct StageArgs {
     double a, b;
     int mode, use_b, use_a;
     int full_rows;      // tout written in whole rows (stage_ghost_cols)
-    const int32_t *gnb;  // 2D halo gather: senders of each block's 9 directions (by hvy id), or null
+    // halo gather, or null.  2D: senders of each block's 9 directions, by hvy
+    // id; 3D: senders of its 6 faces (-1: own ghost nodes), by active position
+    const int32_t *gnb;
 };
 
 struct NoEpilogue {};
@@ -643,11 +717,9 @@ __device__ __forceinline__ int xcd_swizzle(int w, int nw)
 }
 
 // 3D: 256 interior points per workgroup, stencil reads served by L1/L2;
-// XCD: workgroup indices swizzled so that a block's workgroups share an L2;
-// WPE: minimum waves per SIMD of the register allocation (4 spills a few
-// registers to scratch).
-template <int S, bool SKEW, bool FUSED, bool XCD, int WPE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void k_rhs3d(const double *__restrict__ in, double *__restrict__ out,
+// XCD: workgroup indices swizzled so that a block's workgroups share an L2.
+template <int S, bool SKEW, bool FUSED, bool XCD>
+__global__ __launch_bounds__(256) void k_rhs3d(const double *__restrict__ in, double *__restrict__ out,
                                                const double *__restrict__ mask,
                                                const int32_t *__restrict__ act,
                                                const double *__restrict__ x0dx, Geo G, AcmDev a,
@@ -729,119 +801,154 @@ __global__ __launch_bounds__(256) void k_rhs3d_multi(const MPoolDev *__restrict_
 // through z.  The x/y stencils read an LDS copy of the current z-plane slab
 // (interior from the threads' registers, the R-wide x/y ring from global
 // memory); the z stencil reads a per-thread register queue of 2R+1 planes.
-// The next plane's values are fetched before the current one is computed.
+// Everything the next plane needs -- the queue's new plane, the ring, the
+// accumulator and u0 values of the epilogue -- is requested before the
+// current plane is computed, so a plane's memory latency runs under the
+// previous plane's arithmetic.  Two LDS planes (nbuf 2) leave one barrier per
+// plane; one plane (nbuf 1, slabs too wide for two) needs a second one.
 // Every input value is read from memory once (plus the slab ring), except
 // that with zsplit > 1 the z range of a block is cut into zsplit pieces,
 // each with its own workgroups, which read the 2R planes around their cut.
-// WPE: the minimum waves per SIMD the register allocation must allow (1: no
-// constraint; 3 may spill a few registers to scratch).
-template <int S, bool SKEW, bool FUSED, int WPE>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE))) void k_rhs3d_zm(const double *__restrict__ in,
+// Halo: with sa.gnb the values beyond a face of the block come from the
+// interior of the same-level neighbour there (6 ids per block: -x, +x, -y,
+// +y, -z, +z), or from the block's own ghost nodes where the id is -1;
+// without it always from the ghost nodes.  The stencils run along the axes,
+// so edges and corners are not read.
+// Bound by the memory system: over 4096 24^3 blocks (FD4, g 6, middle and
+// outer stages of RK4) 2.26 ms a launch for 9.2 GB = 4.1 TB/s, where a large
+// copy reaches 4.4 (before: 4.34 ms, and 3.30 ms by the flat kernel); over
+// 512 blocks 0.29 ms (0.56, 0.42).
+template <int S, bool SKEW, bool FUSED>
+__global__ __launch_bounds__(512) void k_rhs3d_zm(const double *__restrict__ in,
                                                   double *__restrict__ out,
                                                   const double *__restrict__ mask,
                                                   const int32_t *__restrict__ act,
                                                   const double *__restrict__ x0dx, Geo G, AcmDev a,
-                                                  StageArgs sa, int ysplit, int zsplit)
+                                                  StageArgs sa, int ysplit, int zsplit, int nbuf)
 {
     constexpr int R = Reach<S>::R;
     constexpr int W = 2 * R + 1;
-    constexpr int MAXRING = 4;  // ring elements per thread held in registers
-    extern __shared__ double plane[];
+    extern __shared__ double planes[];
     const int per_block = ysplit * zsplit;
-    const int k = blockIdx.x / per_block;
-    const int rem = blockIdx.x - k * per_block;
+    const int wg = xcd_swizzle((int)blockIdx.x, (int)gridDim.x);
+    const int k = wg / per_block;
+    const int rem = wg - k * per_block;
     const int zpart = rem / ysplit, part = rem - zpart * ysplit;
     const int tz0 = G.bs2 / zsplit, z0 = zpart * tz0, z1 = z0 + tz0;
     const int b = act[k];
     const int ty0 = G.bs1 / ysplit;
     const int y0 = part * ty0;
     const int tid = threadIdx.x;
-    const int ix = tid % G.bs0, iyl = tid / G.bs0, iy = y0 + iyl;
+    const int iyl = tid / G.bs0, ix = tid - iyl * G.bs0, iy = y0 + iyl;
     const int tx = G.bs0 + 2 * R, ty = ty0 + 2 * R, tcs = tx * ty;
-    const size_t zs = (size_t)G.nx * G.ny;
+    const int zs = G.nx * G.ny, cs = (int)G.cs;
     const double *u = in + (size_t)b * G.blk;
-    const size_t col = (size_t)(G.g + iy) * G.nx + (G.g + ix);
-    const int nthr = G.bs0 * ty0;
-    const int ring = 2 * R * (G.bs0 + ty0);  // x/y ring of the slab, without corners
+    // where the values beyond each face are read, relative to their place in
+    // this block's ghost nodes
+    ptrdiff_t fo[6] = {0, 0, 0, 0, 0, 0};
+    if (FUSED && sa.gnb) {
+        const int32_t *nb = sa.gnb + (size_t)k * 6;
+        const ptrdiff_t sh[3] = {G.bs0, (ptrdiff_t)G.bs1 * G.nx, (ptrdiff_t)G.bs2 * zs};
+#pragma unroll
+        for (int f = 0; f < 6; ++f)
+            if (nb[f] >= 0) fo[f] = ((ptrdiff_t)nb[f] - b) * (ptrdiff_t)G.blk + (f & 1 ? -sh[f >> 1] : sh[f >> 1]);
+    }
+    const int col = (G.g + iy) * G.nx + (G.g + ix);
     const double dx0 = x0dx[6 * k + 3], dx1 = x0dx[6 * k + 4], dx2 = x0dx[6 * k + 5];
-    const double inv[3] = {1.0 / dx0, 1.0 / dx1, 1.0 / dx2};
-    const double inv2[3] = {1.0 / (dx0 * dx0), 1.0 / (dx1 * dx1), 1.0 / (dx2 * dx2)};
+    const double inv[3] = {wave_uniform(1.0 / dx0), wave_uniform(1.0 / dx1), wave_uniform(1.0 / dx2)};
+    const double inv2[3] = {wave_uniform(1.0 / (dx0 * dx0)), wave_uniform(1.0 / (dx1 * dx1)),
+                            wave_uniform(1.0 / (dx2 * dx2))};
     const double *mk = mask ? mask + (G.mask_per_block ? (size_t)b * G.mblk : 0) : nullptr;
 
-    // ring element h -> (component, offset in LDS, offset in the block plane)
-    int r_lds[MAXRING];
-    size_t r_glb[MAXRING];
-    int nring = 0;
-    for (int h = tid; h < 4 * ring && nring < MAXRING; h += nthr, ++nring) {
-        const int c = h / ring;
-        const int e = h - c * ring;
+    // thread h holds position h of the slab's x/y ring (without corners; the
+    // host checks that there are no more positions than threads)
+    const bool ringer = tid < 2 * R * (G.bs0 + ty0);
+    int r_lds = 0;
+    const double *r_src = u;
+    if (ringer) {
         int px, py;
-        if (e < 2 * R * G.bs0) {
-            const int row = e / G.bs0;
-            px = R + (e - row * G.bs0);
-            py = row < R ? row : ty0 + row;
-        } else {
-            const int e2 = e - 2 * R * G.bs0;
-            const int kk = e2 % (2 * R);
-            py = R + e2 / (2 * R);
+        ptrdiff_t o = 0;
+        if (tid < 2 * R * G.bs0) {  // rows below and above the slab
+            py = iyl < R ? iyl : ty0 + iyl;
+            px = R + ix;
+            if (iyl < R && part == 0) o = fo[2];
+            if (iyl >= R && part == ysplit - 1) o = fo[3];
+        } else {  // columns left and right
+            const int e = tid - 2 * R * G.bs0, kk = e % (2 * R);
+            py = R + e / (2 * R);
             px = kk < R ? kk : G.bs0 + kk;
+            o = kk < R ? fo[0] : fo[1];
         }
-        r_lds[nring] = c * tcs + py * tx + px;
-        r_glb[nring] = c * G.cs + (size_t)(G.g + y0 - R + py) * G.nx + (G.g - R + px);
+        r_lds = py * tx + px;
+        r_src = u + o + (ptrdiff_t)(G.g + y0 - R + py) * G.nx + (G.g - R + px);
     }
-
+    // the slab's own points of plane iz (-R .. Bs2 + R - 1), component c
+    auto own = [&](int iz, int c) -> double {
+        const double *p = u + (iz < 0 ? fo[4] : iz >= G.bs2 ? fo[5] : (ptrdiff_t)0);
+        return p[c * cs + (G.g + iz) * zs + col];
+    };
+    const int npts = G.bs0 * G.bs1 * G.bs2;
+    const StageBlk SB = FUSED ? stage_blk<4>(sa, b, G.blk, npts) : StageBlk{};
+    double apre[4] = {0, 0, 0, 0}, upre[4] = {0, 0, 0, 0};
     double q[4][W];
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int j = 0; j < 2 * R; ++j) q[c][j] = u[c * G.cs + (size_t)(G.g + z0 - R + j) * zs + col];
-    double nq[4], nr[MAXRING];
+        for (int j = 0; j < 2 * R; ++j) q[c][j] = own(z0 - R + j, c);
+    double nq[4], nr[4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) nq[c] = u[c * G.cs + (size_t)(G.g + z0 + R) * zs + col];
+    for (int c = 0; c < 4; ++c) nq[c] = own(z0 + R, c);
+    if (ringer)
 #pragma unroll
-    for (int j = 0; j < MAXRING; ++j)
-        if (j < nring) nr[j] = u[(size_t)(G.g + z0) * zs + r_glb[j]];
+        for (int c = 0; c < 4; ++c) nr[c] = r_src[c * cs + (G.g + z0) * zs];
 
     const int lc = (iyl + R) * tx + (ix + R);
     for (int iz = z0; iz < z1; ++iz) {
-        const size_t zoff = (size_t)(G.g + iz) * zs;
+        double *plane = planes + (nbuf == 2 && ((iz - z0) & 1) ? 4 * tcs : 0);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             q[c][2 * R] = nq[c];
             plane[c * tcs + lc] = q[c][R];
         }
+        if (ringer)
 #pragma unroll
-        for (int j = 0; j < MAXRING; ++j)
-            if (j < nring) plane[r_lds[j]] = nr[j];
-        if (iz + 1 < z1) {  // prefetch the next plane
-            const size_t zn = zoff + zs;
+            for (int c = 0; c < 4; ++c) plane[c * tcs + r_lds] = nr[c];
+        const int gi = (G.g + iz) * zs + col, pnt = (iz * G.bs1 + iy) * G.bs0 + ix;
+        if constexpr (FUSED) {  // the epilogue's operands
+            if (sa.mode >= 1) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) nq[c] = u[c * G.cs + zn + R * zs + col];
+                for (int c = 0; c < 4; ++c) apre[c] = SB.acc[c * npts + pnt];
+            }
+            if (sa.mode == 1) {
 #pragma unroll
-            for (int j = 0; j < MAXRING; ++j)
-                if (j < nring) nr[j] = u[zn + r_glb[j]];
+                for (int c = 0; c < 4; ++c) upre[c] = SB.u0[c * cs + gi];
+            }
+        }
+        if (iz + 1 < z1) {  // the next plane's values
+#pragma unroll
+            for (int c = 0; c < 4; ++c) nq[c] = own(iz + 1 + R, c);
+            if (ringer)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) nr[c] = r_src[c * cs + (G.g + iz + 1) * zs];
         }
         __syncthreads();
         // x/y from the LDS plane, z from the register queue
         const auto A = [&](int c, int d, int o) -> double {
-            if (d == 2) return q[c][R + o];
+            if (d == 2 || o == 0) return q[c][R + (d == 2 ? o : 0)];
             return plane[c * tcs + lc + o * (d == 0 ? 1 : tx)];
         };
-        const size_t gi = zoff + col;
         double r[4];
         acm_point<3, S, SKEW>(A, inv, inv2, a, mk ? mk + gi : nullptr, G.cs, r);
-        const size_t o = (size_t)b * G.blk + gi;
         if constexpr (FUSED) {
             const double u0c[4] = {q[0][R], q[1][R], q[2][R], q[3][R]};
-            const int npts = G.bs0 * G.bs1 * G.bs2;
-            const StageBlk SB = stage_blk<4>(sa, b, G.blk, npts);
-            stage_epilogue<4>(sa, SB, k, (int)gi, (int)G.cs, (iz * G.bs1 + iy) * G.bs0 + ix, npts, r, u0c, 1);
-            stage_ghost_cols<4>(sa, SB, (int)gi - (G.g + ix), (int)G.cs, ix, G.bs0, G.g);
+            stage_epilogue_pre<4>(sa, SB, k, gi, cs, pnt, npts, r, u0c, 1, apre, upre);
+            stage_ghost_cols<4>(sa, SB, gi - (G.g + ix), cs, ix, G.bs0, G.g);
         } else {
+            double *o = out + (size_t)b * G.blk + gi;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) out[o + c * G.cs] = r[c];
+            for (int c = 0; c < 4; ++c) o[c * cs] = r[c];
         }
-        __syncthreads();
+        if (nbuf == 1) __syncthreads();
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -872,16 +979,52 @@ bool zm_valid(int bs0, int bs1, int scheme, int ys)
     return sizeof(double) * 4 * (bs0 + 2 * R) * (ty0 + 2 * R) <= 64 * 1024;
 }
 
-// y-split of the 3D stage kernel: the pool's tuned value, or the smallest
-// valid split; 0 selects the flat kernel.
+// y-split of the 3D stage kernel: the pool's tuned value, or of the valid
+// splits of at most 256 threads the one that leaves most lanes of a compute
+// unit's 12 resident wavefronts (3 per SIMD) with a column (whole wavefronts,
+// a count that divides 12), the widest slab among equals; 0 selects the flat
+// kernel.
 static int zm_split(const wh_pool *P, const Geo &G, int scheme)
 {
     if (P->k3d_ysplit == 0) return 0;
     if (P->k3d_ysplit > 0 && zm_valid(G.bs0, G.bs1, scheme, P->k3d_ysplit)) return P->k3d_ysplit;
-    for (int ys = 1; ys <= 8; ++ys)
-        if (zm_valid(G.bs0, G.bs1, scheme, ys)) return ys;
-    return 0;
+    int best = 0, most = 0;
+    for (int ys = 1; ys <= 8; ++ys) {
+        if (!zm_valid(G.bs0, G.bs1, scheme, ys)) continue;
+        const int nthr = G.bs0 * (G.bs1 / ys), waves = (nthr + 63) / 64, lanes = 12 / waves * nthr;
+        if (lanes > most) {
+            best = ys;
+            most = lanes;
+        }
+    }
+    return best;
 }
+
+// z-split: the pool's tuned value where it is valid.  With the automatic
+// y-split and no z-split asked for: the FD2 / FD4 stencils without the
+// skew-symmetric products take the largest valid one up to 8 -- short
+// marches even out the last round of workgroups (24^3 blocks, y-split 3:
+// 2335 / 2294 / 2259 us in 1 / 3 / 6 pieces over 4096 blocks, 322 / 300 /
+// 291 us over 512; 20x16x18 over 64 blocks 46 / 20 us in 1 / 3).  The others
+// pay more for the planes read twice (512 blocks: FD6 318 / 330 us in 1 / 2,
+// skew-symmetric FD4 301 / 306 us): the smallest split that gives every
+// compute unit 4 workgroups, else the largest (skew-symmetric FD6, 64 blocks:
+// 67 / 48 / 44 us in 1 / 2 / 4).
+static int zm_zsplit(const wh_pool *P, const Geo &G, const AcmDev &a, int nwg)
+{
+    if (P->k3d_ysplit >= 0 || P->k3d_zsplit != 1)
+        return zm_zvalid(G.bs2, a.scheme, P->k3d_zsplit) ? P->k3d_zsplit : 1;
+    const bool fill_only = a.skew || reach_of(a.scheme) > 2;
+    int best = 1;
+    for (int zs = 1; zs <= 8; ++zs) {
+        if (!zm_zvalid(G.bs2, a.scheme, zs)) continue;
+        best = zs;
+        if (fill_only && (long)nwg * zs >= 4L * P->n_cu) break;
+    }
+    return best;
+}
+
+bool stage_gathers(const wh_pool *P, int scheme) { return P->d.dim == 3 && zm_split(P, make_geo(P), scheme) > 0; }
 
 Geo make_geo(const wh_pool *P)
 {
@@ -960,18 +1103,14 @@ static int dispatch_rhs(wh_pool *P, const AcmDev &a, const double *in, double *o
 #undef L2D
     } else if (const int ys = zm_split(P, G, a.scheme); ys > 0) {
         const int R = reach_of(a.scheme);
-        const int zs = zm_zvalid(G.bs2, a.scheme, P->k3d_zsplit) ? P->k3d_zsplit : 1;
-        const size_t lds = sizeof(double) * 4 * (G.bs0 + 2 * R) * (G.bs1 / ys + 2 * R);
+        const int zs = zm_zsplit(P, G, a, nact * ys);
+        const size_t plane = sizeof(double) * 4 * (G.bs0 + 2 * R) * (G.bs1 / ys + 2 * R);
+        const int nbuf = 2 * plane <= 64 * 1024 ? 2 : 1;
+        const size_t lds = nbuf * plane;
         dim3 grid(nact * ys * zs), blockd(G.bs0 * (G.bs1 / ys));
-#define L3D(SC, SK)                                                                                    \
-    do {                                                                                                \
-        if (P->k3d_waves == 3)                                                                          \
-            hipLaunchKernelGGL((k_rhs3d_zm<SC, SK, FUSED, 3>), grid, blockd, lds, P->stream, in, out, mask, \
-                               act, x0dx, G, a, sa, ys, zs);                                            \
-        else                                                                                            \
-            hipLaunchKernelGGL((k_rhs3d_zm<SC, SK, FUSED, 1>), grid, blockd, lds, P->stream, in, out, mask, \
-                               act, x0dx, G, a, sa, ys, zs);                                            \
-    } while (0)
+#define L3D(SC, SK)                                                                                      \
+    hipLaunchKernelGGL((k_rhs3d_zm<SC, SK, FUSED>), grid, blockd, lds, P->stream, in, out, mask, act, x0dx, G, \
+                       a, sa, ys, zs, nbuf)
         switch (a.scheme * 2 + a.skew) {
         case WH_FD2 * 2: L3D(WH_FD2, false); break;
         case WH_FD2 * 2 + 1: L3D(WH_FD2, true); break;
@@ -987,16 +1126,14 @@ static int dispatch_rhs(wh_pool *P, const AcmDev &a, const double *in, double *o
     } else {
         const int npts = G.bs0 * G.bs1 * G.bs2;
         dim3 grid(nact * ((npts + 255) / 256)), blockd(256);
-#define L3F(SC, SK, X, W)                                                                          \
-    hipLaunchKernelGGL((k_rhs3d<SC, SK, FUSED, X, W>), grid, blockd, 0, P->stream, in, out, mask, act, \
-                       x0dx, G, a, sa)
-#define L3D(SC, SK)                                            \
-    do {                                                        \
-        const bool w4 = P->k3d_waves == 4;                      \
-        if (P->k3d_xcd && w4) L3F(SC, SK, true, 4);             \
-        else if (P->k3d_xcd) L3F(SC, SK, true, 1);              \
-        else if (w4) L3F(SC, SK, false, 4);                     \
-        else L3F(SC, SK, false, 1);                             \
+#define L3D(SC, SK)                                                                                          \
+    do {                                                                                                     \
+        if (P->k3d_xcd)                                                                                      \
+            hipLaunchKernelGGL((k_rhs3d<SC, SK, FUSED, true>), grid, blockd, 0, P->stream, in, out, mask, act, \
+                               x0dx, G, a, sa);                                                              \
+        else                                                                                                 \
+            hipLaunchKernelGGL((k_rhs3d<SC, SK, FUSED, false>), grid, blockd, 0, P->stream, in, out, mask, act, \
+                               x0dx, G, a, sa);                                                              \
     } while (0)
         switch (a.scheme * 2 + a.skew) {
         case WH_FD2 * 2: L3D(WH_FD2, false); break;
@@ -1009,7 +1146,6 @@ static int dispatch_rhs(wh_pool *P, const AcmDev &a, const double *in, double *o
         case WH_FD6 * 2 + 1: L3D(WH_FD6, true); break;
         default: set_error("unknown scheme"); return WH_E_ARG;
         }
-#undef L3F
 #undef L3D
     }
     WH_HIP(hipGetLastError());
