@@ -845,12 +845,15 @@ int decompose_full_tree(Tree &T, const wh_adapt_params &p)
     if (p.decompose_branch == 1) leaf_first = true;
     if (p.decompose_branch == 2) leaf_first = false;
     int level = T.max_level();
-    std::vector<int> all(n_leaf);
+    // hvy_tmp = hvy_block for the leaves that are not flagged: the first
+    // round copies the flagged ones as it decomposes them, and its sync reads
+    // those in hvy_block (SRC_NOT_FLAG); without a round all are copied here
+    std::vector<int> later;
     for (int i = 0; i < n_leaf; ++i) {
-        all[i] = i;
         if (T.b[i].level == level || leaf_first) T.b[i].status = -1;
+        if (T.b[i].status != -1 || level < p.jmin) later.push_back(i);
     }
-    if (int rc = dev_blocks(T, WOP_COPY, A_U, A_T, hvy_of(T, all))) return rc;
+    if (int rc = dev_blocks(T, WOP_COPY, A_U, A_T, hvy_of(T, later))) return rc;
     if (int rc = init_full_tree(T, p.jmin)) return rc;
     const int g_this = std::max(std::abs(w.hd_lo), w.gd_hi);
     int it = 0;
@@ -869,10 +872,8 @@ int decompose_full_tree(Tree &T, const wh_adapt_params &p)
             if (T.b[i].level == p.jmax && p.force_maxlevel_dealiasing) dea.push_back(i);
             else dec.push_back(i);
         }
-        std::vector<int> both(dec);
-        both.insert(both.end(), dea.begin(), dea.end());
-        if (int rc = dev_blocks(T, WOP_COPY, A_U, A_T, hvy_of(T, both))) return rc;
-        if (int rc = dev_blocks(T, WOP_FWT, A_T, A_U, hvy_of(T, dec))) return rc;
+        if (int rc = dev_blocks(T, WOP_COPY_FWT, A_U, A_T, hvy_of(T, dec))) return rc;
+        if (int rc = dev_blocks(T, WOP_COPY, A_U, A_T, hvy_of(T, dea))) return rc;
         if (int rc = dev_blocks(T, WOP_FILTER, A_T, A_U, hvy_of(T, dea))) return rc;
         if (p.use_ce)
             if (int rc = ce_modify(T, CE_REF, 0, -1, true, true)) return rc;

@@ -331,7 +331,9 @@ int run_boxes(wh_pool *P, int array, int src_array, const std::vector<wh_box> &b
 void noalloc_setup(int dev);
 int run_detail(wh_pool *P, int array, const std::vector<int32_t> &ids, const int32_t *groups,
                std::vector<double> &detail);
-enum { WOP_FWT = 0, WOP_IWT = 1, WOP_FILTER = 2, WOP_COPY = 3 };
+// WOP_COPY_FWT: the blocks of src_array copied to dst_array, whole, and
+// decomposed in src_array
+enum { WOP_FWT = 0, WOP_IWT = 1, WOP_FILTER = 2, WOP_COPY = 3, WOP_COPY_FWT = 4 };
 // per-box component maxima (|v|, SCs zeroed with zero_sc, sqrt(v*v) for
 // grouped components with sqrt_groups): out[k*neq + c]
 // Reductions launched into a caller's device range d_out (no copy, no

@@ -543,6 +543,299 @@ __global__ __launch_bounds__(256) void k_wring(double *__restrict__ arr, const i
     }
 }
 
+// ---------------------------------------------------------------------------
+// Transforms with the chains known at compile time.  The offsets of the
+// chains of CDFXY follow from X and Y alone (which taps of HR and of the
+// lifting stencil vanish); the host compares them with the term tables of
+// the pool's filters (fixed_chain) and passes the coefficients.  The sums are
+// those of the tables, term by term.
+// ---------------------------------------------------------------------------
+constexpr int FIXED_MAX = 13;  // terms of the longest of these chains (and their window)
+struct FixedChain {
+    int n[2], off[2][FIXED_MAX];
+    int lo, hi;  // the reach of both
+};
+struct FixedCoef {
+    double c[2][FIXED_MAX];
+};
+constexpr bool odd_tap(int order, int i) { return (i & 1) && i < order && i > -order; }
+// is HD(i) a non-zero tap (setup: delta + 1/2 HR * h, h the odd taps of order Y)?
+constexpr bool hd_tap(int X, int Y, int i)
+{
+    if (i == 0) return true;
+    for (int j = 1 - X; Y > 0 && j < X; ++j)
+        if ((j == 0 || odd_tap(X, j)) && odd_tap(Y, i - j)) return true;
+    return false;
+}
+template <int OP, int X, int Y>
+constexpr FixedChain fixed_chain()
+{
+    FixedChain F{};
+    auto add = [&](int par, int off) {
+        F.off[par][F.n[par]++] = off;
+        if (off < F.lo) F.lo = off;
+        if (off > F.hi) F.hi = off;
+    };
+    const int m = X + Y;  // beyond every tap
+    if (OP == WOP_FWT) {
+        for (int i = -m; i <= m; ++i)
+            if (hd_tap(X, Y, i)) add(0, i);
+        for (int i = -m; i <= m; ++i)
+            if (i == 0 || odd_tap(X, i)) add(1, i);
+    } else {
+        add(0, 0);
+        for (int i = -m; Y > 0 && i <= m; ++i)
+            if ((i & 1) && hd_tap(X, Y, i)) add(0, i);
+        if (Y == 0) add(1, 0);
+        for (int i = -m; i <= m; ++i)
+            if (odd_tap(X, i)) add(1, i);
+        if (Y > 0) add(1, 0);
+        for (int i = -m; Y > 0 && i <= m; ++i)
+            if (i != 0 && !(i & 1) && hd_tap(X, Y, i)) add(1, i);
+    }
+    return F;
+}
+
+template <int OP, int X, int Y, int PAR, class F>
+__device__ __forceinline__ double fixed_sum(const FixedCoef &C, F at)
+{
+    constexpr FixedChain K = fixed_chain<OP, X, Y>();
+    double s = at(K.off[PAR][0]) * C.c[PAR][0];
+#pragma unroll
+    for (int k = 1; k < K.n[PAR]; ++k) s = s + at(K.off[PAR][k]) * C.c[PAR][k];
+    return s;
+}
+
+// The x and y passes of a transform on one z plane of one component of one
+// block (2D: the whole transform).  The plane goes to LDS, the x pass runs
+// over the interior columns of the rows [g - ext, g + Bs1 + ext) into a second
+// LDS plane, the y pass over the interior rows from there; what is written
+// is what the separate passes write: y values in the interior rows, x values
+// in the extended ones.  Points of one class (even or odd along the pass) fill
+// whole wavefronts, so a wavefront sums one chain.
+// copy: the source block as it was, whole (then src and dst may be the same
+// array: a plane is written only after it is in LDS).
+// init_copy: the points no pass reaches take the source's values.
+// Bound by memory: it replaces chains whose offsets were read from a table
+// (and took a 64-bit address per term): 4096 2D blocks, CDF44, 16^2 44 -> 34
+// us a call, 24^2 81 -> 51.
+struct XfGeo {
+    size_t blk_in, blk_out, blk_copy, cs;
+    int nx, ny, nz, neq, g, bs0, bs1, ext, z0, z1;
+    FastDiv xa, xb, dx;  // by the x classes' sizes and by Bs0
+};
+template <int OP, int X, int Y>
+__global__ __launch_bounds__(256) void k_xyplane(const double *in, double *out, double *copy,
+                                                 const int32_t *__restrict__ ids, XfGeo G, int init_copy, FixedCoef C)
+{
+    extern __shared__ double sp[];
+    const int nxy = G.nx * G.ny, tid = threadIdx.x;
+    double *S = sp, *D = sp + nxy;  // D: the extended rows of the interior columns
+    const int bc = (int)blockIdx.x / G.nz, z = (int)blockIdx.x - bc * G.nz;
+    const int k = bc / G.neq, c = bc - k * G.neq;
+    const size_t b = (size_t)ids[k], zo = (size_t)c * G.cs + (size_t)z * nxy;
+    const double *src = in + b * G.blk_in + zo;
+    double *dst = out + b * G.blk_out + zo;
+    double *cpy = copy ? copy + b * G.blk_copy + zo : nullptr;
+    const bool pass = z >= G.z0 && z < G.z1;  // uniform
+    if (!pass && !cpy && !init_copy) return;
+    const int rows = G.bs1 + 2 * G.ext;
+    for (int i0 = tid; i0 < nxy; i0 += 4 * 256) {
+        double v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (i0 + j * 256 < nxy) v[j] = src[i0 + j * 256];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = i0 + j * 256;
+            if (i >= nxy) break;
+            S[i] = v[j];
+            if (cpy) cpy[i] = v[j];
+            if (init_copy) {
+                const int y = i / G.nx, x = i - y * G.nx - G.g;
+                const int r = y - (G.g - G.ext);
+                if (!pass || x < 0 || x >= G.bs0 || r < 0 || r >= rows) dst[i] = v[j];
+            }
+        }
+    }
+    if (!pass) return;
+    __syncthreads();
+    const int xA = (G.bs0 + 1) / 2, xB = G.bs0 / 2;
+    const int xpa = (xA * rows + 63) & ~63, xtot = xpa + xB * rows;
+    for (int e = tid; e < xtot; e += 256) {
+        const bool cb = __builtin_amdgcn_readfirstlane(e >= xpa ? 1 : 0);
+        const int r = cb ? e - xpa : e;
+        if (!cb && e >= xA * rows) continue;
+        const int i1 = fdiv(r, cb ? G.xb : G.xa), j = r - i1 * (cb ? xB : xA);
+        const int i0 = 2 * j + (cb ? 1 : 0);
+        const int q = (G.g - G.ext + i1) * G.nx + G.g + i0;
+        const double *sq = S + q;
+        auto at = [&](int off) { return sq[off]; };
+        const double v = cb ? fixed_sum<OP, X, Y, 1>(C, at) : fixed_sum<OP, X, Y, 0>(C, at);
+        D[i1 * G.bs0 + i0] = v;
+        if (i1 < G.ext || i1 >= G.ext + G.bs1) dst[q] = v;
+    }
+    __syncthreads();
+    const int yA = (G.bs1 + 1) / 2, yB = G.bs1 / 2;
+    const int pa = (yA * G.bs0 + 63) & ~63, tot = pa + yB * G.bs0;
+    for (int e = tid; e < tot; e += 256) {
+        const bool cb = __builtin_amdgcn_readfirstlane(e >= pa ? 1 : 0);
+        const int r = cb ? e - pa : e;
+        if (!cb && e >= yA * G.bs0) continue;
+        const int j = fdiv(r, G.dx), i0 = r - j * G.bs0, y = 2 * j + (cb ? 1 : 0);
+        const double *dq = D + (G.ext + y) * G.bs0 + i0;
+        const int nb = G.bs0;
+        auto at = [&](int off) { return dq[off * nb]; };
+        dst[(G.g + y) * G.nx + G.g + i0] = cb ? fixed_sum<OP, X, Y, 1>(C, at) : fixed_sum<OP, X, Y, 0>(C, at);
+    }
+}
+
+// A 3D transform of one component of one block in one workgroup, in one sweep
+// over its z planes: per plane the x and y passes of k_xyplane; each thread
+// owns one (x, y) point and keeps its last K.hi - K.lo + 1 y values in
+// registers, from which the z chain of plane z - K.hi follows.  Every value
+// is read once and written once (k_xyplane and k_zcolumn write and read the
+// interior planes again for z).  Bound by the latency of a plane: the next
+// plane is requested before the current one is worked on, and what a plane
+// yields is stored just before that request, so that waiting for the loads
+// (which waits for the stores before them too) finds both done.
+// copy, init_copy: as in k_xyplane.
+constexpr int XYZ_PRE = 4;  // plane values per thread (the host checks that they suffice)
+template <int OP, int X, int Y>
+__global__ __launch_bounds__(1024) void k_xyz(const double *in, double *out, double *copy,
+                                              const int32_t *__restrict__ ids, XfGeo G, int bs2, int init_copy,
+                                              FixedCoef C)
+{
+    constexpr FixedChain K = fixed_chain<OP, X, Y>();
+    constexpr int WN = K.hi - K.lo + 1;
+    extern __shared__ double sp[];
+    const int nxy = G.nx * G.ny, tid = threadIdx.x, nt = blockDim.x;
+    double *S = sp, *D = sp + nxy;
+    const int k = (int)blockIdx.x / G.neq, c = (int)blockIdx.x - k * G.neq;
+    const size_t b = (size_t)ids[k];
+    const double *src = in + b * G.blk_in + (size_t)c * G.cs;
+    double *dst = out + b * G.blk_out + (size_t)c * G.cs;
+    double *cpy = copy ? copy + b * G.blk_copy + (size_t)c * G.cs : nullptr;
+    const int rows = G.bs1 + 2 * G.ext;
+    int outside = 0;  // bit j: this thread's j-th plane value lies where no pass writes
+    if (init_copy)
+        for (int j = 0; j < XYZ_PRE; ++j) {
+            const int i = tid + j * nt, y = i / G.nx, x = i - y * G.nx - G.g, r = y - (G.g - G.ext);
+            if (i < nxy && (x < 0 || x >= G.bs0 || r < 0 || r >= rows)) outside |= 1 << j;
+        }
+    if (cpy || init_copy)
+        for (int z = 0; z < G.nz; ++z) {  // the planes outside the passes
+            if (z >= G.z0 && z < G.z1) continue;
+            for (int i = tid; i < nxy; i += nt) {
+                const double v = src[z * nxy + i];
+                if (cpy) cpy[z * nxy + i] = v;
+                if (init_copy) dst[z * nxy + i] = v;
+            }
+        }
+    // this thread's (x, y) point: even rows first, then odd rows
+    const int yA = (G.bs1 + 1) / 2, pa = (yA * G.bs0 + 63) & ~63;
+    const bool odd = __builtin_amdgcn_readfirstlane(tid >= pa ? 1 : 0);
+    const int r = odd ? tid - pa : tid, jy = fdiv(r, G.dx), x = r - jy * G.bs0, y = 2 * jy + (odd ? 1 : 0);
+    const bool have = odd ? jy < G.bs1 / 2 : jy < yA;
+    const double *dq = D + (have ? (G.ext + y) * G.bs0 + x : G.ext * G.bs0);
+    const int q = have ? (G.g + y) * G.nx + G.g + x : -1;
+    const int xA = (G.bs0 + 1) / 2, xB = G.bs0 / 2;
+    const int xpa = (xA * rows + 63) & ~63, xtot = xpa + xB * rows;
+    double w[WN], pre[XYZ_PRE], yv = 0.0, zv = 0.0;
+    auto load = [&](int z) {
+#pragma unroll
+        for (int j = 0; j < XYZ_PRE; ++j) pre[j] = src[z * nxy + min(tid + j * nt, nxy - 1)];
+    };
+    // what plane z yielded: x values in the extended rows (still in D), y
+    // values in the extended planes, the z values of plane z - K.hi
+    auto store = [&](int z) {
+        double *dz = dst + (ptrdiff_t)z * nxy;
+        for (int e = tid; e < 2 * G.ext * G.bs0; e += nt) {
+            const int i = fdiv(e, G.dx), xx = e - i * G.bs0, i1 = i < G.ext ? i : G.bs1 + i;
+            dz[(G.g - G.ext + i1) * G.nx + G.g + xx] = D[i1 * G.bs0 + xx];
+        }
+        if (q < 0) return;
+        if (z < G.g || z >= G.g + bs2) dz[q] = yv;
+        const int zz = z - K.hi;
+        if (zz >= G.g && zz < G.g + bs2) dst[zz * nxy + q] = zv;
+    };
+    load(G.z0);
+    for (int z = G.z0; z < G.z1; ++z) {
+#pragma unroll
+        for (int j = 0; j < XYZ_PRE; ++j) {
+            const int i = tid + j * nt;
+            if (i < nxy) {
+                S[i] = pre[j];
+                if (cpy) cpy[z * nxy + i] = pre[j];
+                if (outside >> j & 1) dst[z * nxy + i] = pre[j];
+            }
+        }
+        if (z > G.z0) store(z - 1);
+        load(min(z + 1, G.z1 - 1));
+        __syncthreads();
+        for (int e = tid; e < xtot; e += nt) {
+            const bool cb = __builtin_amdgcn_readfirstlane(e >= xpa ? 1 : 0);
+            const int rr = cb ? e - xpa : e;
+            if (!cb && e >= xA * rows) continue;
+            const int i1 = fdiv(rr, cb ? G.xb : G.xa), j = rr - i1 * (cb ? xB : xA);
+            const int i0 = 2 * j + (cb ? 1 : 0);
+            const double *sq = S + (G.g - G.ext + i1) * G.nx + G.g + i0;
+            auto at = [&](int off) { return sq[off]; };
+            D[i1 * G.bs0 + i0] = cb ? fixed_sum<OP, X, Y, 1>(C, at) : fixed_sum<OP, X, Y, 0>(C, at);
+        }
+        __syncthreads();
+        const int nb = G.bs0;
+        auto at = [&](int off) { return dq[off * nb]; };
+        yv = odd ? fixed_sum<OP, X, Y, 1>(C, at) : fixed_sum<OP, X, Y, 0>(C, at);
+#pragma unroll
+        for (int t = 0; t + 1 < WN; ++t) w[t] = w[t + 1];
+        w[WN - 1] = yv;
+        auto az = [&](int off) { return w[off - K.lo]; };
+        zv = (z - K.hi - G.g) & 1 ? fixed_sum<OP, X, Y, 1>(C, az) : fixed_sum<OP, X, Y, 0>(C, az);
+    }
+    store(G.z1 - 1);
+}
+
+// The z pass of a transform, in place: one thread per interior (x, y) column
+// of a component, marching in z with the chain's window of planes in
+// registers; four planes are requested at a time, each before any output at
+// or above it is written.
+template <int OP, int X, int Y>
+__global__ __launch_bounds__(256) void k_zcolumn(double *__restrict__ arr, const int32_t *__restrict__ ids, int wpb,
+                                                 size_t blk, size_t cs, int nx, int nxy, int neq, int g, int bs0,
+                                                 int bs1, int bs2, FixedCoef C)
+{
+    constexpr FixedChain K = fixed_chain<OP, X, Y>();
+    constexpr int WN = K.hi - K.lo + 1;
+    const PtIdx I = pt_index(wpb, neq);
+    if (I.t >= bs0 * bs1) return;
+    const int y = I.t / bs0, x = I.t - y * bs0;
+    double *col = arr + (size_t)ids[I.k] * blk + (size_t)I.c * cs + (size_t)g * nxy + (g + y) * nx + g + x;
+    const int last = bs2 - 1 + K.hi;
+    double w[WN], f[4];
+#pragma unroll
+    for (int t = 0; t + 1 < WN; ++t) w[t] = col[(K.lo + t) * nxy];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f[j] = col[min(K.hi + j, last) * nxy];
+    for (int z = 0; z < bs2; z += 4) {
+        double v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[j] = f[j];
+            f[j] = col[min(z + 4 + K.hi + j, last) * nxy];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            w[WN - 1] = v[j];
+            auto at = [&](int off) { return w[off - K.lo]; };
+            const double s = j & 1 ? fixed_sum<OP, X, Y, 1>(C, at) : fixed_sum<OP, X, Y, 0>(C, at);
+            if (z + j < bs2) col[(z + j) * nxy] = s;
+#pragma unroll
+            for (int t = 0; t + 1 < WN; ++t) w[t] = w[t + 1];
+        }
+    }
+}
+
 // Whole listed blocks (all components, contiguous per block) copied in
 // 16-byte words where every block offset and the length are even, in
 // doubles otherwise.
@@ -972,12 +1265,101 @@ int launch_sepxy(wh_pool *P, const double *in, size_t blk_in, double *out, size_
     return WH_OK;
 }
 
+// do the chains of the table have exactly these offsets?
+bool same_chain(const TermTable &T, const FixedChain &F)
+{
+    if (T.from_zero) return false;
+    for (int par = 0; par < 2; ++par) {
+        if (T.n[par] != F.n[par]) return false;
+        for (int k = 0; k < T.n[par]; ++k)
+            if (T.off[par][k] != F.off[par][k] || T.brk[par][k]) return false;
+    }
+    return true;
+}
+
+// The transform by k_xyplane and, in 3D, k_zcolumn, where its chains are
+// known and the block fits (two LDS planes; item counts below 2^16).  *done
+// says whether it was launched.  copy: see k_xyplane (blk_copy its block
+// length), or null.
+template <int OP, int X, int Y>
+int launch_xform_xy(wh_pool *P, const double *in, size_t blk_in, double *out, size_t blk_out, double *copy,
+                    size_t blk_copy, int nb, const TermTable &T, int ext, bool init_copy, bool *done)
+{
+    constexpr FixedChain K = fixed_chain<OP, X, Y>();
+    static_assert(K.hi >= 1 && K.lo <= -1, "a z pass reads planes beyond its outputs");
+    *done = false;
+    if (!same_chain(T, K)) return WH_OK;
+    const int dim = P->d.dim, g = P->d.g, bs0 = P->d.bs[0], bs1 = P->d.bs[1], bs2 = dim == 3 ? P->d.bs[2] : 1;
+    const int rows = bs1 + 2 * ext, nxy = P->nx * P->ny, nz = dim == 3 ? P->nz : 1;
+    // the passes stay in the block: chains reach at most ext <= g
+    if (ext > g || std::max(K.hi, -K.lo) > ext) return WH_OK;
+    const size_t lds = sizeof(double) * (nxy + rows * bs0);
+    if (lds > 64 * 1024 || nxy + 128 >= (1 << 16)) return WH_OK;
+    const int wpb = (bs0 * bs1 + 255) / 256;
+    WH_CHECK((size_t)nb * P->d.neq * std::max(nz, wpb) < (1u << 31), WH_E_ARG,
+             "wavelet transform: too many blocks in one launch");
+    *done = true;
+    if (nb <= 0) return WH_OK;
+    const XfGeo G{blk_in, blk_out, blk_copy, P->cs, P->nx, P->ny, nz, P->d.neq, g, bs0, bs1, ext,
+                  dim == 3 ? g - ext : 0, dim == 3 ? g + bs2 + ext : 1, fast_div((bs0 + 1) / 2),
+                  fast_div(std::max(bs0 / 2, 1)), fast_div(bs0)};
+    FixedCoef C{};
+    for (int par = 0; par < 2; ++par)
+        for (int k = 0; k < T.n[par]; ++k) C.c[par][k] = T.c[par][k];
+    // 3D in one sweep where a workgroup has a thread per (x, y) point and its
+    // march through z is worth it: at least 4 workgroups per compute unit, the
+    // longer filters, no rows to write whole.  Sweep against plane and column
+    // kernel, CDF44: 512 blocks of 24^3 548 / 679 us, of 20^3 391 / 476,
+    // 1024 of 16^3 505 / 618, 256 of 24^3 309 / 324, but 64 of 24^3 78 / 59;
+    // CDF22, 256 of 24^3: 179 / 134; CDF40 reconstruction (whole rows), 512 of
+    // 24^3: 479 / 346.
+    const int items = (((bs1 + 1) / 2 * bs0 + 63) & ~63) + bs1 / 2 * bs0, nt = (items + 63) & ~63;
+    if (dim == 3 && X >= 4 && !init_copy && nt <= 1024 && nxy <= XYZ_PRE * nt &&
+        (long)nb * P->d.neq >= 4L * P->n_cu) {
+        hipLaunchKernelGGL((k_xyz<OP, X, Y>), dim3((unsigned)(nb * P->d.neq)), dim3(nt), lds, P->stream, in, out, copy,
+                           P->ws.cur_ids, G, bs2, init_copy ? 1 : 0, C);
+        WH_HIP(hipGetLastError());
+        return WH_OK;
+    }
+    hipLaunchKernelGGL((k_xyplane<OP, X, Y>), dim3((unsigned)(nb * P->d.neq * nz)), dim3(256), lds, P->stream, in, out,
+                       copy, P->ws.cur_ids, G, init_copy ? 1 : 0, C);
+    if (dim == 3)
+        hipLaunchKernelGGL((k_zcolumn<OP, X, Y>), dim3((unsigned)(nb * P->d.neq * wpb)), dim3(256), 0, P->stream, out,
+                           P->ws.cur_ids, wpb, blk_out, P->cs, P->nx, nxy, P->d.neq, g, bs0, bs1, bs2, C);
+    WH_HIP(hipGetLastError());
+    return WH_OK;
+}
+
+template <int OP>
+int launch_xform(wh_pool *P, const double *in, size_t blk_in, double *out, size_t blk_out, double *copy,
+                 size_t blk_copy, int nb, const TermTable &T, int ext, bool init_copy, bool *done)
+{
+#define LX(XX, YY)                                                                                                   \
+    return launch_xform_xy<OP, XX, YY>(P, in, blk_in, out, blk_out, copy, blk_copy, nb, T, ext, init_copy, done)
+    switch (P->ws.w.X * 10 + P->ws.w.Y) {
+    case 20: LX(2, 0);
+    case 22: LX(2, 2);
+    case 40: LX(4, 0);
+    case 42: LX(4, 2);
+    case 44: LX(4, 4);
+    case 60: LX(6, 0);
+    case 62: LX(6, 2);
+    }
+#undef LX
+    *done = false;
+    return WH_OK;
+}
+
 // Three separable passes (x over an extended row range, then y, then z) of
 // the chains T: x reads `in` and writes `out`; y and z work in place on
 // `out`, a column at a time.
+template <int OP>
 int separable(wh_pool *P, const double *in, size_t blk_in, double *out, size_t blk_out, int nb,
               const TermTable &T, int ext, bool init_copy = false)
 {
+    bool done = false;
+    if (int rc = launch_xform<OP>(P, in, blk_in, out, blk_out, nullptr, 0, nb, T, ext, init_copy, &done)) return rc;
+    if (done) return WH_OK;
     const int g = P->d.g, dim = P->d.dim;
     const int B0 = P->d.bs[0], B1 = P->d.bs[1], B2 = dim == 3 ? P->d.bs[2] : 1;
     const int zlo = dim == 3 ? g - ext : 0, zn = dim == 3 ? B2 + 2 * ext : 1;
@@ -1142,10 +1524,20 @@ int run_blocks_op(wh_pool *P, int op, int src_array, int dst_array, const std::v
     const wh_wavelet &w = P->ws.w;
     WH_CHECK(op == WOP_COPY || P->d.g >= w.g, WH_E_ARG, "wavelet op: too few ghost nodes for the wavelet");
     if (op == WOP_COPY) return launch_copy_blocks(P, in, blk_in, out, blk_out, n);
+    if (op == WOP_COPY_FWT) {
+        const TermTable T = fwt_terms(w);
+        const int ext = std::max(w.hd_hi, w.gd_hi);
+        double *u = array_ptr(P, src_array, nullptr, nullptr);
+        bool done = false;
+        if (int rc = launch_xform<WOP_FWT>(P, u, blk_in, u, blk_in, out, blk_out, n, T, ext, false, &done)) return rc;
+        if (done) return WH_OK;
+        if (int rc = launch_copy_blocks(P, u, blk_in, out, blk_out, n)) return rc;
+        return separable<WOP_FWT>(P, out, blk_out, u, blk_in, n, T, ext);
+    }
     if (op == WOP_FWT)
-        return separable(P, in, blk_in, out, blk_out, n, fwt_terms(w), std::max(w.hd_hi, w.gd_hi));
+        return separable<WOP_FWT>(P, in, blk_in, out, blk_out, n, fwt_terms(w), std::max(w.hd_hi, w.gd_hi));
     if (op == WOP_IWT)  // CDFX0 starts from a copy of the whole block
-        return separable(P, in, blk_in, out, blk_out, n, iwt_terms(w), std::max(w.hr_hi, w.gr_hi), !w.lifted);
+        return separable<WOP_IWT>(P, in, blk_in, out, blk_out, n, iwt_terms(w), std::max(w.hr_hi, w.gr_hi), !w.lifted);
     if (op == WOP_FILTER) return filter_passes(P, in, blk_in, out, blk_out, n);
     set_error("wavelet op: unknown op");
     return WH_E_ARG;
@@ -1725,7 +2117,7 @@ int wh_fwt_threshold_noalloc(wh_pool *pool, int src_array, int dst_array, const 
     const int32_t *saved = P->ws.cur_ids;
     P->ws.cur_ids = d_ids;
     const wh::DetailArgs D = wh::detail_args(P, groups);
-    int rc = wh::separable(P, in, blk_in, out, blk_out, n, wh::fwt_terms(w), std::max(w.hd_hi, w.gd_hi));
+    int rc = wh::separable<wh::WOP_FWT>(P, in, blk_in, out, blk_out, n, wh::fwt_terms(w), std::max(w.hd_hi, w.gd_hi));
     if (!rc) rc = wh::launch_detail(P, out, blk_out, d_ids, n, D, d_det);
     P->ws.cur_ids = saved;
     if (rc) return rc;
