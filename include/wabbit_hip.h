@@ -250,12 +250,7 @@ int wh_batch_time_stage_kernel(wh_batch *batch, const wh_acm_params *p, const do
                                int reps, double *ms, int *blocks);
 int wh_batch_synchronize(wh_batch *batch);
 /* The batch's 2D stage kernel (no counterpart in the reference):
- * WH_TUNE_K2D_STAGE 0 = one block per workgroup at a time, the first
- * point's operands loaded before the tile barrier; 1 = software pipelined
- * (the next block's metadata and halo tile in flight while a block is
- * computed; used where every tile is at most 32 x 32, i.e. Bs <= 28 with
- * FD4); 2 = 0 without the early loads; 3 / 4 = 2 with its registers bounded
- * for 6 / 8 waves per SIMD.  All give the same results bit for bit. */
+ * WH_TUNE_K2D_STAGE takes 0 to 4, without effect (there is one kernel). */
 int wh_batch_set_tuning(wh_batch *batch, int key, int value);
 int wh_batch_get_tuning(wh_batch *batch, int key, int *value);
 
@@ -530,11 +525,8 @@ int wh_set_tables_from_forests(wh_pool *pool, wh_forest *const *forests, int n, 
  * build of each 3D kernel, whose registers allow 3 to 5 waves per SIMD).
  * WH_TUNE_K3D_XCD (default 0): 1 remaps the flat 3D kernel's workgroups so
  * that those of one block run on one XCD (one L2).
- * WH_TUNE_K2D_STAGE: 2D stage kernel variant: 0 one workgroup per block;
- * 1 (default) the same, loading the mask and stage operands of each
- * thread's first point before the halo-tile barrier; 2, 3, 4 a persistent
- * kernel with 2, 4, 8 workgroups per compute unit that loads the next
- * block's halo tile while computing the current one (where the tile fits).
+ * WH_TUNE_K2D_STAGE (default 1): 0 to 4, without effect (there is one 2D
+ * stage kernel; its split of a block into slabs follows from the block size).
  * Every variant computes the same values bit for bit.
  * WH_TUNE_GATHER (default 1): where the RHS ghost-patch table of a 2D pool
  * consists of same-level copies only (a uniform grid) that cover the halo

@@ -94,28 +94,6 @@ static bool fused_ok(const double *bt, int nrows)
     return true;
 }
 
-// The halo-gather table of the fused 2D stages (WH_TUNE_GATHER), or null:
-// the RHS patch table holds same-level copies only, at least as deep as the
-// stencil reach, and every active block has the senders of all 8
-// directions (checked once per topology version).
-static const int32_t *gather_table(wh_pool *P, const AcmDev &a)
-{
-    const PatchSet &ps = P->ps[0];
-    if (!P->gather || P->d.dim != 2 || !ps.gather_ok || !ps.d_gnb || ps.gather_depth < reach_of(a.scheme))
-        return nullptr;
-    if (P->gather_topo != P->topo_version) {
-        bool all = P->nact > 0;
-        for (int k = 0; k < P->nact && all; ++k) {
-            const int32_t *row = &ps.h_gnb[(size_t)P->h_active[k] * 9];
-            for (int d = 0; d < 9 && all; ++d)
-                if (d != 4 && row[d] < 0) all = false;
-        }
-        P->gather_all = all;
-        P->gather_topo = P->topo_version;
-    }
-    return P->gather_all ? ps.d_gnb : nullptr;
-}
-
 // grow a device buffer to at least n elements (contents are not kept);
 // callers synchronise the stream first
 template <class T>
@@ -255,16 +233,51 @@ static int build_faces(wh_pool *P, int R)
     return upload_staged(P, F.d_chunks, F.h_chunks.data(), sizeof(SyncChunk) * F.h_chunks.size());
 }
 
+// The face table of a 2D pool whose RHS patches are same-level copies only
+// (set_patch_runs: gather_ok), at least as deep as the reach R, where every
+// active block has the senders of all 8 directions: then every face is
+// gathered, of the state too, and no patch is left.
+static int build_faces_2d(wh_pool *P, int R)
+{
+    FaceGather &F = P->faces;
+    const PatchSet &ps = P->ps[0];
+    F.reach = R;
+    F.any = ps.gather_depth >= R;
+    for (int k = 0; k < P->nact && F.any; ++k) {
+        const int32_t *row = &ps.h_gnb[(size_t)P->h_active[k] * 9];
+        for (int d = 0; d < 9; ++d)
+            if (d != 4 && row[d] < 0) F.any = false;
+    }
+    if (!F.any) return WH_OK;
+    F.h_kept.clear();
+    F.h_face.resize((size_t)P->nact * 4);
+    for (int k = 0; k < P->nact; ++k) {
+        const int32_t *row = &ps.h_gnb[(size_t)P->h_active[k] * 9];
+        const int at[4] = {3, 5, 1, 7};
+        for (int f = 0; f < 4; ++f) F.h_face[(size_t)k * 4 + f] = row[at[f]];
+    }
+    if (F.h_face.size() > F.cap_face) WH_HIP(hipStreamSynchronize(P->stream));
+    if (int rc = grow_dev(F.d_face, F.cap_face, F.h_face.size())) return rc;
+    return upload_staged(P, F.d_face, F.h_face.data(), sizeof(int32_t) * F.h_face.size());
+}
+
+// do the fused stages of this pool use a face table where there is one?
+static bool gathers(const wh_pool *P, const AcmDev &a)
+{
+    if (!P->gather || P->nact == 0 || P->ps[0].n == 0) return false;
+    return P->d.dim == 2 ? P->ps[0].gather_ok : stage_gathers(P, a.scheme);
+}
+
 // Brings the face table up to date for the fused stages of this scheme (a
 // host-to-device copy where it changed, so before any stream capture).
 static int update_faces(wh_pool *P, const AcmDev &a)
 {
-    if (!P->gather || !stage_gathers(P, a.scheme) || P->nact == 0 || P->ps[0].n == 0) return WH_OK;
+    if (!gathers(P, a)) return WH_OK;
     FaceGather &F = P->faces;
     const int R = reach_of(a.scheme);
     if (F.topo == P->topo_version && F.reach == R) return WH_OK;
     if (F.topo == P->topo_version) P->topo_version++;  // captured graphs hold the other reach's table
-    if (int rc = build_faces(P, R)) return rc;
+    if (int rc = P->d.dim == 2 ? build_faces_2d(P, R) : build_faces(P, R)) return rc;
     F.topo = P->topo_version;
     return WH_OK;
 }
@@ -273,8 +286,7 @@ static int update_faces(wh_pool *P, const AcmDev &a)
 static const FaceGather *face_table(const wh_pool *P, const AcmDev &a)
 {
     const FaceGather &F = P->faces;
-    const bool on = P->gather && stage_gathers(P, a.scheme) && F.any && F.topo == P->topo_version &&
-                    F.reach == reach_of(a.scheme);
+    const bool on = gathers(P, a) && F.any && F.topo == P->topo_version && F.reach == reach_of(a.scheme);
     return on ? &F : nullptr;
 }
 
@@ -289,9 +301,9 @@ static int sync_kept(wh_pool *P, const FaceGather &F, double *arr)
 }
 
 // one step of the fused path; dt is taken from the device scalar DS_DT, or
-// per block from dtb (block groups).  With the 2D halo-gather table no ghost
-// fill is launched: every stage reads its blocks' halos from the
-// neighbours' interiors of its input array.  With a 3D face table the state
+// per block from dtb (block groups).  With a 2D face table no ghost fill is
+// launched: every stage reads its blocks' halos from the neighbours'
+// interiors of its input array.  With a 3D face table the state
 // gets its ghost fill as without it (its ghost nodes are the caller's); of
 // the fills of the stage inputs in the work slots only the kept patches run.
 static int fused_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
@@ -302,17 +314,18 @@ static int fused_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
     double *acc = array_ptr(P, WH_WORK + 0, nullptr, nullptr);
     double *T[2] = {array_ptr(P, WH_WORK + 1, nullptr, nullptr),
                     array_ptr(P, WH_WORK + 2, nullptr, nullptr)};
-    const int32_t *gnb = gather_table(P, a);
     const FaceGather *fg = face_table(P, a);
-    // the ghost fill (timed as a sync launch); nothing at all with gather
+    const bool of_state = P->d.dim == 2;  // whether the first stage, too, uses the face table
+    // the ghost fill (timed as a sync launch)
     auto sync = [&](double *arr) {
-        if (gnb || (fg && arr != S && fg->h_kept.empty())) return (int)WH_OK;
-        return timed(P, 1, [&] { return fg && arr != S ? sync_kept(P, *fg, arr) : wh::launch_sync(P, 0, arr, -1); });
+        const bool faces = fg && (of_state || arr != S);
+        if (faces && fg->h_kept.empty()) return (int)WH_OK;
+        return timed(P, 1, [&] { return faces ? sync_kept(P, *fg, arr) : wh::launch_sync(P, 0, arr, -1); });
     };
     auto launch_fused_stage = [&](wh_pool *Q, const AcmDev &aa, const double *tin, double *tout, const double *u0,
                                   double *ac, double *sout, int mode, double acoef, double bcoef, const double *db) {
         return wh::launch_fused_stage(Q, aa, tin, tout, u0, ac, sout, mode, acoef, bcoef, db,
-                                      gnb ? gnb : fg && tin != S ? fg->d_face : nullptr);
+                                      fg && (of_state || tin != S) ? fg->d_face : nullptr);
     };
     int rc;
     if ((rc = sync(S))) return rc;
@@ -455,7 +468,6 @@ static void free_patchset(PatchSet &ps)
     if (ps.d_recv_off) (void)hipFree(ps.d_recv_off);
     if (ps.d_recv_ids) (void)hipFree(ps.d_recv_ids);
     if (ps.d_chunks) (void)hipFree(ps.d_chunks);
-    if (ps.d_gnb) (void)hipFree(ps.d_gnb);
     ps = PatchSet{};
 }
 
@@ -798,11 +810,6 @@ static int set_patch_runs(wh_pool *P, int sync_case, const PatchRun *runs, int n
         if (int rc = grow_dev(ps.d_chunks, ps.cap_chunks, ps.h_chunks.size())) return rc;
         if (int rc = upload_staged(P, ps.d_chunks, ps.h_chunks.data(), sizeof(SyncChunk) * ps.h_chunks.size()))
             return rc;
-        if (ps.gather_ok) {
-            if (ps.h_gnb.size() > ps.cap_gnb) WH_HIP(hipStreamSynchronize(P->stream));
-            if (int rc = grow_dev(ps.d_gnb, ps.cap_gnb, ps.h_gnb.size())) return rc;
-            if (int rc = upload_staged(P, ps.d_gnb, ps.h_gnb.data(), sizeof(int32_t) * ps.h_gnb.size())) return rc;
-        }
         if (int rc = upload_staged(P, ps.d_patches, ps.host.data(), sizeof(wh_patch) * npatch)) return rc;
         if (int rc = upload_staged(P, ps.d_recv_off, ps.h_recv_off.data(), sizeof(int32_t) * ps.h_recv_off.size()))
             return rc;
@@ -1218,9 +1225,8 @@ int wh_time_stage_kernel(wh_pool *P, const wh_acm_params *p, int reps, double *m
     double *acc = array_ptr(P, WH_WORK + 0, nullptr, nullptr), *tout = array_ptr(P, WH_WORK + 1, nullptr, nullptr),
            *sout = array_ptr(P, WH_WORK + 2, nullptr, nullptr);
     // the four stages of classic RK4 (first, two middle, last), reading the
-    // state and writing only work slots; with the halo-gather table the
-    // steps use, the launches gather their halos the same way
-    const int32_t *gnb = gather_table(P, a);
+    // state and writing only work slots; with the face table the steps use,
+    // the launches gather their halos the same way
     if (int rc = update_faces(P, a)) return rc;
     const FaceGather *fg = face_table(P, a);
     auto rk4 = [&]() -> int {
@@ -1230,7 +1236,7 @@ int wh_time_stage_kernel(wh_pool *P, const wh_acm_params *p, int reps, double *m
             if (int rc = launch_fused_stage(P, a, P->block, mode[j] == 2 ? nullptr : tout,
                                             mode[j] == 1 ? P->block : nullptr, acc, mode[j] == 2 ? sout : nullptr,
                                             mode[j], ca[j], cb[j], nullptr,
-                                            gnb ? gnb : fg && j > 0 ? fg->d_face : nullptr))
+                                            fg && (P->d.dim == 2 || j > 0) ? fg->d_face : nullptr))
                 return rc;
         return WH_OK;
     };
@@ -1255,9 +1261,9 @@ int wh_autotune(wh_pool *P, const wh_acm_params *p, int reps, int *best_value, d
     WH_CHECK(P->nact > 0, WH_E_STATE, "autotune needs an active list");
     WH_CHECK(!P->timing, WH_E_STATE, "disable kernel timing before autotuning");
     reps = std::max(1, std::min(reps, 100));
-    // 3D: the flat kernel and the z-marching (y-split, z-split) pairs; 2D:
-    // the load order of the mask and stage operands.  The variant value is
-    // reported in best_value (3D: the y-split; the z-split is set too).
+    // 3D: the flat kernel and the z-marching (y-split, z-split) pairs; 2D has
+    // one kernel.  The variant value is reported in best_value (3D: the
+    // y-split; the z-split is set too).
     struct Var {
         int v, zs, waves, xcd;
     };
@@ -1270,7 +1276,7 @@ int wh_autotune(wh_pool *P, const wh_acm_params *p, int reps, int *best_value, d
                 if (zm_valid(P->d.bs[0], P->d.bs[1], p->scheme, ys) && zm_zvalid(P->d.bs[2], p->scheme, zs))
                     cand.push_back({ys, zs, 1, 0});
     } else {
-        for (int v = 0; v <= 4; ++v) cand.push_back({v, 1, 1, 0});
+        cand.push_back({P->k2d_stage, 1, 1, 0});
     }
     int &knob = three ? P->k3d_ysplit : P->k2d_stage;
     const AcmDev a = make_acm_dev(p);

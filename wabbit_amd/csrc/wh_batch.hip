@@ -38,7 +38,7 @@ struct wh_batch {
     // group (capacity cap_grp), counts ([0] entries, [s] chunks and [3 + s]
     // patches of sync stage s)
     MPoolDev *d_pools = nullptr;
-    wh::MEnt *d_ents = nullptr;  // entry records, one per slot of the pools
+    wh::MEnt *d_ents = nullptr;  // item records, for every slot of the pools
     double *d_dtg = nullptr;
     AcmDev *d_gacm = nullptr;
     int64_t *d_tot = nullptr;
@@ -56,13 +56,7 @@ struct wh_batch {
     int nchunk = 1, grid_stage = 0, grid_sync = 0;
     int n_ent_last = 0;
     int sout_sel = 0;  // the last stage's output array (0: the state; 3 while timing)
-    // 2D stage kernel (WH_TUNE_K2D_STAGE): 0 one block per workgroup at a
-    // time with the first point's operands loaded before the tile barrier;
-    // 1 software-pipelined (used where every tile is at most 32 x 32); 2 as
-    // 0 without the early loads; 3 / 4 as 2 with registers for 6 / 8 waves
-    // per SIMD
-    int k2d = 0;
-    bool pipe_ok = false;  // the last step's tiles fit the pipelined kernel
+    int k2d = 0;  // WH_TUNE_K2D_STAGE as set (no effect)
     int full_rows = 0;     // the last step's stages write their outputs in whole rows
 };
 
@@ -89,14 +83,8 @@ void free_graph(wh_batch *B)
     B->graph = nullptr;
 }
 
-bool pipe_on(const wh_batch *B) { return B->dim == 2 && B->k2d == 1 && B->pipe_ok; }
-
-// the launcher's kernel choice (0: the default kernel)
-int k2d_sel(const wh_batch *B) { return B->dim != 2 ? 0 : B->k2d == 1 ? (pipe_on(B) ? 1 : 0) : B->k2d; }
-
-// persistent stage-kernel grids, multiples of 8 (one per XCD); the pipelined
-// kernel holds more registers, so its grid stays resident at 4 per CU
-int stage_grid(const wh_batch *B) { return B->dim == 2 ? (pipe_on(B) ? 4 : 8) * B->n_cu : 16 * B->n_cu; }
+// persistent stage-kernel grids, multiples of 8 (one per XCD)
+int stage_grid(const wh_batch *B) { return (B->dim == 2 ? 8 : 16) * B->n_cu; }
 
 // the RK stage sequence of the fused path (runge_kutta_generic.f90:63-154 with
 // the stage-j RHS and its accumulation fused, as wh_rk_step path 2)
@@ -125,7 +113,7 @@ int launch_sequence(wh_batch *B, const wh_acm_params &p, const double *bt, int n
         ms.full_rows = B->full_rows;
         return wh::launch_stage_multi(B->stream, B->dim, p.scheme, p.skew_symmetry ? 1 : 0, 1, B->d_pools, np,
                                       B->d_ents, B->d_dtg, B->d_gacm, B->d_tot, ms, B->lds, B->grid_stage,
-                                      B->nchunk, k2d_sel(B));
+                                      B->nchunk);
     };
     // arrays: 0 state, 1 accumulator (work 0), 2 / 3 ping-pong stage inputs
     if (int rc = sync(0)) return rc;
@@ -218,7 +206,11 @@ int wh_batch_create(wh_batch **out, wh_pool *const *pools, int npools)
     if ((e = hipMalloc(&B->d_tot, sizeof(int64_t) * 7)) != hipSuccess) return fail(e);
     if ((e = hipMalloc(&B->d_pools, sizeof(MPoolDev) * npools)) != hipSuccess) return fail(e);
     size_t slots = 0;
-    for (int i = 0; i < npools; ++i) slots += (size_t)pools[i]->d.nb_max;
+    for (int i = 0; i < npools; ++i) {
+        const wh_pool_desc &d = pools[i]->d;
+        const int ty0 = wh::slab_rows(d.bs[0], d.bs[1]);
+        slots += (size_t)d.nb_max * (dim == 2 ? (d.bs[1] + ty0 - 1) / ty0 : 1);
+    }
     if ((e = hipMalloc(&B->d_ents, sizeof(wh::MEnt) * slots)) != hipSuccess) return fail(e);
     *out = B;
     return WH_OK;
@@ -261,10 +253,9 @@ int wh_batch_rk_step(wh_batch *B, const wh_acm_params *p, const double *bt, int 
     size_t lds = 0;
     int nchunk = 1;
     const int R = p->scheme == WH_FD2 ? 1 : p->scheme == WH_FD4 ? 2 : 3;
-    int goff = 0, nent = 0;
+    int goff = 0, nent = 0, nitem = 0;  // block groups, blocks, items
     double step_bytes = 0.0;  // one block of every entry
     int64_t tot[7] = {0, 0, 0, 0, 0, 0, 0};
-    bool pipe_ok = true;
     for (int i = 0; i < npools; ++i) {
         wh_pool *P = B->pools[i];
         WH_CHECK(P->nact == (int)P->h_active.size() && (P->nact == 0 || P->ngrp > 0), WH_E_STATE,
@@ -299,7 +290,9 @@ int wh_batch_rk_step(wh_batch *B, const wh_acm_params *p, const double *bt, int 
         m.grp = P->d_grp;
         m.pt = ps.d_patches;
         m.ch = ps.d_chunks;
-        m.ent0 = nent;
+        m.ent0 = nitem;
+        m.ty0 = B->dim == 2 ? wh::slab_rows(P->d.bs[0], P->d.bs[1]) : P->d.bs[1];
+        m.nslab = (P->d.bs[1] + m.ty0 - 1) / m.ty0;
         m.goff = goff;
         for (int st = 1; st <= 3; ++st) {
             const int a = ps.n ? ps.stage_begin[st] : 0, b = ps.n ? ps.stage_begin[st + 1] : 0;
@@ -319,17 +312,18 @@ int wh_batch_rk_step(wh_batch *B, const wh_acm_params *p, const double *bt, int 
             }
         }
         if (P->nact > 0) {
-            if (std::max(P->d.bs[0], P->d.bs[1]) + 2 * R > 32) pipe_ok = false;
-            if (B->dim == 2)
-                lds = std::max(lds, sizeof(double) * 3 * (P->d.bs[0] + 2 * R) * (P->d.bs[1] + 2 * R));
-            else
+            if (B->dim == 2) {
+                WH_CHECK(wh::tile2d_ok(P->d.bs[0], P->d.bs[1], R), WH_E_ARG, "2D block tile exceeds LDS");
+                lds = std::max(lds, sizeof(double) * 3 * (P->d.bs[0] + 2 * R) * (m.ty0 + 2 * R));
+            } else
                 nchunk = std::max(nchunk, (P->d.bs[0] * P->d.bs[1] * P->d.bs[2] + 255) / 256);
         }
         nent += P->nact;
+        nitem += P->nact * m.nslab;
         goff += P->ngrp;
         step_bytes += (double)P->nact * sizeof(double) * (double)m.G.blk;
     }
-    tot[0] = nent;
+    tot[0] = nitem;
     if (gacm.empty()) {
         gacm.push_back(wh::make_acm_dev(p));
         dtg.push_back(0.0);
@@ -382,7 +376,6 @@ int wh_batch_rk_step(wh_batch *B, const wh_acm_params *p, const double *bt, int 
     // launch geometry
     B->lds = lds;
     B->nchunk = nchunk;
-    B->pipe_ok = pipe_ok;
     B->full_rows = wh::stage_full_rows(1.0, step_bytes) ? 1 : 0;
     B->grid_stage = stage_grid(B);
     B->grid_sync = 4 * B->n_cu;
@@ -394,7 +387,6 @@ int wh_batch_rk_step(wh_batch *B, const wh_acm_params *p, const double *bt, int 
         key.push_back((double)lds);
         key.push_back(nchunk);
         key.push_back(npools);
-        key.push_back(k2d_sel(B));
         key.push_back(B->full_rows);
         if (!B->gexec || B->graph_version != ver || key != B->graph_key) {
             free_graph(B);
@@ -449,7 +441,7 @@ int wh_batch_time_stage_kernel(wh_batch *B, const wh_acm_params *p, const double
         m.full_rows = B->full_rows;
         return wh::launch_stage_multi(B->stream, B->dim, p->scheme, p->skew_symmetry ? 1 : 0, 1, B->d_pools,
                                       (int)B->pools.size(), B->d_ents, B->d_dtg, B->d_gacm, B->d_tot, m, B->lds,
-                                      stage_grid(B), B->nchunk, k2d_sel(B));
+                                      stage_grid(B), B->nchunk);
     };
     // the last step's entry records (rebuilt from its descriptors)
     int rc = wh::launch_entries(B->stream, B->d_pools, (int)B->pools.size(), B->d_tot, B->d_ents, 2 * B->n_cu);

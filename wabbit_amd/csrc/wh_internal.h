@@ -70,7 +70,7 @@ struct SyncChunk {
 // pool's own device tables -- active list, origin/spacing and block group
 // per active position, the RHS ghost-patch table with its slot prefix sum --
 // and the pool's place in the launch: its first entry (entries are the
-// pools' active lists one after the other), its first block group, and per
+// pools' active lists one after the other, nslab per block), its first block group, and per
 // sync stage s its patch range [p0[s], p1[s]) and chunk range [c0[s],
 // c1[s]), and where these start in the launch: its first chunk s0[s] among
 // the stage's chunks and its first patch q0[s] among the stage's patches
@@ -85,18 +85,19 @@ struct MPoolDev {
     const int32_t *grp;
     const wh_patch *pt;
     const SyncChunk *ch;
-    int ent0, goff;
+    int ent0, goff, nslab, ty0;  // items per block and rows of each (3D: 1, Bs1)
     int p0[3], p1[3], c0[3], c1[3];
     int64_t s0[3], q0[3];
 };
 
-// Entry k of a multi-pool launch, resolved once per step (launch_entries):
-// its pool, hvy id, block group in the launch (goff + grp) and position in
-// the pool's active list.  The stage kernels read one record per block
-// instead of searching the pools and then reading the active list and the
-// group table one after the other.
+// Item k of a multi-pool launch, resolved once per step (launch_entries): a
+// slab of a block in 2D (slab_rows; rows [y0, y0 + ty0) of its interior), a
+// block in 3D: its pool, hvy id, block group in the launch (goff + grp) and
+// position in the pool's active list.  The stage kernels read one record per
+// item instead of searching the pools and then reading the active list and
+// the group table one after the other.
 struct MEnt {
-    int32_t pool, b, g, j;
+    int32_t pool, b, g, j, y0, ty0;
 };
 
 // The RK stage of a multi-pool fused stage launch: input / output array
@@ -164,8 +165,6 @@ struct PatchSet {
     bool gather_ok = false;
     int gather_depth = 0;
     std::vector<int32_t> h_gnb;
-    int32_t *d_gnb = nullptr;
-    size_t cap_gnb = 0;
     int stage_begin[5] = {0, 0, 0, 0, 0};  // stage s (1..3): patches [stage_begin[s], stage_begin[s+1])
     int chunk_begin[5] = {0, 0, 0, 0, 0};  // and chunks [chunk_begin[s], chunk_begin[s+1])
     int n = 0, nrecv = 0;
@@ -237,15 +236,8 @@ struct wh_pool {
     int k3d_zsplit = 1;
     int k3d_waves = 1;  // WH_TUNE_K3D_WAVES as set (no effect)
     int k3d_xcd = 0;    // 1: the flat 3D kernel's workgroups swizzled per XCD
-    // tuning of the 2D stage kernel: 0 plain, 1 mask and epilogue operands
-    // loaded before the tile barrier, 2..4 persistent pipelined kernel with
-    // 2, 4, 8 workgroups per CU
-    int k2d_stage = 1;
-    // WH_TUNE_GATHER, and whether the current tables allow it (checked once
-    // per topology version: every active block has its 8 senders)
-    int gather = 1;
-    uint64_t gather_topo = ~0ull;
-    bool gather_all = false;
+    int k2d_stage = 1;  // WH_TUNE_K2D_STAGE as set (no effect)
+    int gather = 1;  // WH_TUNE_GATHER
     int n_cu = 256;  // compute units of the pool's device
     int device = 0;  // the device the pool lives on
     // wavelet transforms / adapt_tree
@@ -277,8 +269,7 @@ int launch_combine(wh_pool *P, double *out, const double *base, int nterms,
 int launch_dt(wh_pool *P, const AcmDev &a);
 int launch_maxabs(wh_pool *P, const double *in);
 // dtb: per active-list position dt (block groups), or null for the pool's DS_DT
-// gnb: 2D: the halo-gather table (the ghost fill skipped), 3D: the face table
-// (FaceGather) of the z-marching kernel, or null
+// gnb: the face table (FaceGather; 3D: of the z-marching kernel), or null
 int launch_fused_stage(wh_pool *P, const AcmDev &a, const double *tin, double *tout,
                        const double *u0, double *acc, double *sout, int mode, double acoef,
                        double bcoef, const double *dtb, const int32_t *gnb = nullptr);
@@ -386,8 +377,7 @@ Geo make_geo(const wh_pool *P);
 // multi-pool launches (independent forests of a batch, wh_batch.hip)
 // d_tot: [0] entries of the launch, [s] chunks of sync stage s (1..3), [3 + s]
 // patches of sync stage s; dtg /
-// gacm: dt and constants per block group of the launch; pipe: the 2D
-// software-pipelined kernel (tile widths and heights <= 32)
+// gacm: dt and constants per block group of the launch
 // a run of ghost patches (set_patch_table takes several, one after the other)
 struct PatchRun {
     const wh_patch *p;
@@ -401,10 +391,12 @@ int launch_entries(hipStream_t stream, const MPoolDev *d_pools, int npools, cons
                    int grid);
 int launch_stage_multi(hipStream_t stream, int dim, int scheme, int skew, int xcd, const MPoolDev *d_pools,
                        int npools, const MEnt *d_ents, const double *d_dtg, const AcmDev *d_gacm,
-                       const int64_t *d_tot, const MStage &ms, size_t lds, int grid, int nchunk, int pipe = 0);
+                       const int64_t *d_tot, const MStage &ms, size_t lds, int grid, int nchunk);
 int launch_sync_multi(hipStream_t stream, const MPoolDev *d_pools, int npools, int sel, int stage,
                       const int64_t *d_tot, int grid, int dim);
 int reach_of(int scheme);
+int slab_rows(int bs0, int bs1);
+bool tile2d_ok(int bs0, int bs1, int R);
 bool zm_valid(int bs0, int bs1, int scheme, int ys);
 bool zm_zvalid(int bs2, int scheme, int zs);
 

@@ -92,81 +92,37 @@ __device__ __forceinline__ double wave_uniform(double v)
     return x.d;
 }
 
-// ACM right-hand side at one point (RHS_2D_acm / RHS_3D_acm).  A(c, d, o) is
-// component c of the state at offset o along direction d from the point.
-// mk: mask component 0 at this point (components mcs apart) or null.
-template <int DIM, int S, bool SKEW, class ACC>
-__device__ __forceinline__ void acm_point_all(const ACC &A, const double *inv, const double *inv2,
-                                          const AcmDev &a, const double *__restrict__ mk,
-                                          ptrdiff_t mcs, double *r)
-{
-    double uv[DIM + 1];
-    double du[DIM + 1][DIM];
-#pragma unroll
-    for (int c = 0; c <= DIM; ++c) {
-        uv[c] = A(c, 0, 0);
-#pragma unroll
-        for (int d = 0; d < DIM; ++d)
-            du[c][d] = d1<S>([&](int o) { return A(c, d, o); }, inv[d]);
-    }
-    double chi = 0.0;
-    if (a.penal && mk) {
-        const int color = (int)mk[4 * mcs];
-        chi = mk[0] * (color == 0 ? 0.0 : a.Cinv);
-    }
-#pragma unroll
-    for (int c = 0; c < DIM; ++c) {
-        double lap = d2<S>([&](int o) { return A(c, 0, o); }, inv2[0]);
-#pragma unroll
-        for (int d = 1; d < DIM; ++d)
-            lap = lap + d2<S>([&](int o) { return A(c, d, o); }, inv2[d]);
-        double t;
-        if constexpr (SKEW) {
-            double sum = d1p<S>([&](int o) { return A(c, 0, o); },
-                                [&](int o) { return A(0, 0, o); }, inv[0]);
-#pragma unroll
-            for (int d = 1; d < DIM; ++d)
-                sum = sum + d1p<S>([&](int o) { return A(c, d, o); },
-                                   [&](int o) { return A(d, d, o); }, inv[d]);
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) sum = sum + uv[d] * du[c][d];
-            t = -(0.5 * sum);
-        } else {
-            t = -(uv[0] * du[c][0]);
-#pragma unroll
-            for (int d = 1; d < DIM; ++d) t = t - uv[d] * du[c][d];
-        }
-        t = t - du[DIM][c];
-        t = t + a.nu * lap;
-        if (a.penal && mk) t = t + (-(chi * (uv[c] - mk[(1 + c) * mcs])));
-        r[c] = t;
-    }
-    double div = du[0][0];
-#pragma unroll
-    for (int d = 1; d < DIM; ++d) div = div + du[d][d];
-    r[DIM] = -(a.c02 * div) - a.gamma_p * uv[DIM];
-    if (a.sponge && mk) {
-        const double spo = mk[5 * mcs] * a.Csp_inv;
-#pragma unroll
-        for (int c = 0; c < DIM; ++c) r[c] = r[c] - (uv[c] - a.ums[c]) * spo;
-        r[DIM] = r[DIM] - uv[DIM] * spo;
-    }
-}
+// the mask components of a point, if it has any: in memory (components cs
+// apart) or in registers
+struct MaskMem {
+    const double *p;
+    ptrdiff_t cs;
+    __device__ __forceinline__ bool on() const { return p != nullptr; }
+    __device__ __forceinline__ double operator()(int i) const { return p[i * cs]; }
+};
+struct MaskReg {
+    double v[6];
+    bool has;
+    __device__ __forceinline__ bool on() const { return has; }
+    __device__ __forceinline__ double operator()(int i) const { return v[i]; }
+};
 
-// The same values with the components one after the other, so that few
-// derivatives are live at once (3D FD4: 90 instead of 144 registers in the
-// flat kernel, 147 instead of 201 in the z-marching one).
-template <int DIM, int S, bool SKEW, class ACC>
-__device__ __forceinline__ void acm_point_seq(const ACC &A, const double *inv, const double *inv2,
-                                          const AcmDev &a, const double *__restrict__ mk,
-                                          ptrdiff_t mcs, double *r)
+// ACM right-hand side at one point (RHS_2D_acm / RHS_3D_acm).  A(c, d, o) is
+// component c of the state at offset o along direction d from the point;
+// mk: the point's mask (MaskMem or MaskReg).
+// The components one after the other, so that few derivatives are live at
+// once (3D FD4: 90 instead of 144 registers in the flat kernel, 147 instead of
+// 201 in the z-marching one; 2D FD4 75 instead of 96).
+template <int DIM, int S, bool SKEW, class ACC, class MASK>
+__device__ __forceinline__ void acm_point(const ACC &A, const double *inv, const double *inv2, const AcmDev &a,
+                                              const MASK &mk, double *r)
 {
     double chi = 0.0, spo = 0.0;
-    if (a.penal && mk) {
-        const int color = (int)mk[4 * mcs];
-        chi = mk[0] * (color == 0 ? 0.0 : a.Cinv);
+    if (a.penal && mk.on()) {
+        const int color = (int)mk(4);
+        chi = mk(0) * (color == 0 ? 0.0 : a.Cinv);
     }
-    if (a.sponge && mk) spo = mk[5 * mcs] * a.Csp_inv;
+    if (a.sponge && mk.on()) spo = mk(5) * a.Csp_inv;
     double div = 0.0;
 #pragma unroll
     for (int c = 0; c < DIM; ++c) {
@@ -196,24 +152,14 @@ __device__ __forceinline__ void acm_point_seq(const ACC &A, const double *inv, c
         }
         t = t - d1<S>([&](int o) { return A(DIM, c, o); }, inv[c]);
         t = t + a.nu * lap;
-        if (a.penal && mk) t = t + (-(chi * (uc - mk[(1 + c) * mcs])));
-        if (a.sponge && mk) t = t - (uc - a.ums[c]) * spo;
+        if (a.penal && mk.on()) t = t + (-(chi * (uc - mk(1 + c))));
+        if (a.sponge && mk.on()) t = t - (uc - a.ums[c]) * spo;
         r[c] = t;
         div = c == 0 ? du[0] : div + du[c];
     }
     const double p = A(DIM, 0, 0);
     r[DIM] = -(a.c02 * div) - a.gamma_p * p;
-    if (a.sponge && mk) r[DIM] = r[DIM] - p * spo;
-}
-
-// 2D: all derivatives first (registers are no limit there, and the loads
-// are all requested at once); 3D: component by component
-template <int DIM, int S, bool SKEW, class ACC>
-__device__ __forceinline__ void acm_point(const ACC &A, const double *inv, const double *inv2, const AcmDev &a,
-                                          const double *__restrict__ mk, ptrdiff_t mcs, double *r)
-{
-    if constexpr (DIM == 2) acm_point_all<DIM, S, SKEW>(A, inv, inv2, a, mk, mcs, r);
-    else acm_point_seq<DIM, S, SKEW>(A, inv, inv2, a, mk, mcs, r);
+    if (a.sponge && mk.on()) r[DIM] = r[DIM] - p * spo;
 }
 
 // accessor over one strided storage: base = component 0 of the point,
@@ -228,6 +174,18 @@ struct StridedAcc {
         return base[c * cs + o * s[d]];
     }
 };
+
+// Workgroups are dispatched to the 8 XCDs (each with its own L2) round-robin:
+// workgroup w runs on XCD w % 8.  The swizzle gives XCD x the consecutive
+// logical indices [start(x), start(x) + count(x)), so the workgroups of one
+// block share an L2 instead of being spread over all eight.  A permutation
+// of [0, nw) for any nw.
+__device__ __forceinline__ int xcd_swizzle(int w, int nw)
+{
+    constexpr int NX = 8;
+    const int q = nw / NX, r = nw - q * NX, x = w % NX;
+    return x * q + min(x, r) + w / NX;
+}
 
 // Runge-Kutta epilogue of the fused stage kernel.
 //   mode 0 (first stage): u0 = input state; acc = u0 + (dt*b)*k; tout = u0 + (dt*a)*k
@@ -247,8 +205,8 @@ struct StageArgs {
     double a, b;
     int mode, use_b, use_a;
     int full_rows;      // tout written in whole rows (stage_ghost_cols)
-    // halo gather, or null.  2D: senders of each block's 9 directions, by hvy
-    // id; 3D: senders of its 6 faces (-1: own ghost nodes), by active position
+    // halo gather: the senders of each block's 4 (2D) or 6 faces by active
+    // position (-1: own ghost nodes), or null
     const int32_t *gnb;
 };
 
@@ -340,138 +298,187 @@ __device__ __forceinline__ void stage_ghost_cols(const StageArgs &sa, const Stag
     }
 }
 
-// stage_ghost_cols for every interior row of a 2D block, by the whole
+// stage_ghost_cols for the rows [y0, y0 + ty0) of a 2D block, by the whole
 // workgroup after its points (no per-point registers live meanwhile)
 template <int NC>
-__device__ __forceinline__ void stage_ghost_cols_2d(const StageArgs &sa, const StageBlk &B, const Geo &G)
+__device__ __forceinline__ void stage_ghost_cols_2d(const StageArgs &sa, const StageBlk &B, const Geo &G, int y0,
+                                                    int ty0)
 {
     if (!sa.full_rows || sa.mode == 2 || !sa.use_a) return;
     const int w = 2 * G.g, cs = (int)G.cs;
-    for (int i = threadIdx.x; i < G.bs1 * w; i += blockDim.x) {
+    for (int i = threadIdx.x; i < ty0 * w; i += blockDim.x) {
         const int r = i / w, x = i - r * w;
-        const int o = (G.g + r) * G.nx + (x < G.g ? x : G.bs0 + x);
+        const int o = (G.g + y0 + r) * G.nx + (x < G.g ? x : G.bs0 + x);
 #pragma unroll
         for (int c = 0; c < NC; ++c) B.tout[o + c * cs] = 0.0;
     }
 }
 
-// 2D: one workgroup per block, the (Bs+2R)^2 x 3 halo tile staged in LDS.
-// With PRE each thread loads the mask and, for the fused stages, the acc /
-// u0 values of its first point into registers before the tile barrier, so
-// that these reads overlap the tile load instead of following it.
-// rhs2d_block is the work of one workgroup on block b (active position k):
-// shared by the one-pool kernel and the multi-pool kernel.  mk: the mask of
-// block b or null.
-// LOADED: the caller has already put the tile in LDS (and synchronised).
-template <int S, bool SKEW, bool FUSED, bool PRE, bool LOADED = false>
-__device__ __forceinline__ void rhs2d_block(double *tile, const double *__restrict__ in, double *__restrict__ out,
-                                            const double *__restrict__ mk, int b, int k,
-                                            const double *__restrict__ x0dx, const Geo &G, const AcmDev &a,
-                                            const StageArgs &sa)
+// 2D: a slab of ty0 rows of one block per workgroup (a thread per point where
+// the slab has no more points than threads), its points and the R layers
+// around them staged in LDS -- the edges only: the stencils run along the
+// axes.  Everything a thread's first point needs is requested before the tile
+// barrier: its own value and one halo position (per component), the mask and
+// the accumulator and u0 values of the fused stages.
+// Bound by the launch for small grids (4.3 us for 256 blocks of 16^2, before
+// 6.2; 4.3 for 64 of 32^2, before 14.9), by memory for large ones: 4096 blocks
+// of 24^2 38.6 us = 7.1 TB/s from the cache-resident arrays with FD4 (before
+// 74), 52 us with FD6 (102): one slab's loads are few enough to be in flight
+// together, and no index is divided per tile element.
+// rhs2d_slab is the work of one workgroup on the rows [y0, y0 + ty0) of block
+// b (active position k), shared by the one-pool and the multi-pool kernel.
+// mk: the mask of block b or null.  faces: the ids of the same-level
+// neighbours (-x, +x, -y, +y) whose interior holds the values beyond the
+// block's faces, or null (and -1) for the block's own ghost nodes.
+template <int S, bool SKEW, bool FUSED>
+__device__ __forceinline__ void rhs2d_slab(double *tile, const double *__restrict__ in, double *__restrict__ out,
+                                           const double *__restrict__ mk, int b, int k, int y0, int ty0,
+                                           const double *__restrict__ x0dx, const int32_t *__restrict__ faces,
+                                           const Geo &G, const AcmDev &a, const StageArgs &sa)
 {
-    static_assert(!(PRE && LOADED), "the operand prefetch belongs to the tile load");
     constexpr int R = Reach<S>::R;
-    const int tx = G.bs0 + 2 * R, ty = G.bs1 + 2 * R, tcs = tx * ty;
-    const int npts = G.bs0 * G.bs1;
-    const size_t base = (size_t)b * G.blk;
-    const int p0 = threadIdx.x;
-    const int cs = (int)G.cs;
-    const StageBlk SB = FUSED ? stage_blk<3>(sa, b, G.blk, npts) : StageBlk{};
-    double mpre[6] = {0, 0, 0, 0, 0, 0}, apre[3] = {0, 0, 0}, upre[3] = {0, 0, 0};
-    if constexpr (PRE) {
-        if (p0 < npts) {
-            const int iy = p0 / G.bs0, ix = p0 - iy * G.bs0;
-            const int gi = (G.g + iy) * G.nx + (G.g + ix);
-            if (mk) {
-#pragma unroll
-                for (int c = 0; c < 6; ++c)
-                    if (c != 3) mpre[c] = mk[c * G.cs + gi];  // component 3 (u_s,z) is 3D only
-            }
-            if (FUSED && sa.mode >= 1) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) apre[c] = SB.acc[c * npts + p0];
-                if (sa.mode == 1) {
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) upre[c] = SB.u0[c * cs + gi];
-                }
-            }
-        }
-    }
-    if constexpr (!LOADED) {
-        const double *u = in + (size_t)b * G.blk;
-        if (FUSED && sa.gnb) {
-            // the halo from the neighbours' interiors (same-level senders, the
-            // values the ghost fill would copy): tile point (x, y) relative to
-            // the interior lies in direction (dx, dy) of the block
-            const int32_t *nb = sa.gnb + (size_t)b * 9;
-            for (int i = threadIdx.x; i < 3 * tcs; i += blockDim.x) {
-                const int c = i / tcs, rr = i - c * tcs;
-                const int y = rr / tx - R, x = rr - (y + R) * tx - R;
-                const int dx = x < 0 ? -1 : (x >= G.bs0 ? 1 : 0), dy = y < 0 ? -1 : (y >= G.bs1 ? 1 : 0);
-                const double *src = (dx | dy) ? in + (size_t)nb[(dy + 1) * 3 + dx + 1] * G.blk : u;
-                tile[i] = src[c * G.cs + (size_t)(G.g + y - dy * G.bs1) * G.nx + (G.g + x - dx * G.bs0)];
-            }
-        } else {
-            for (int i = threadIdx.x; i < 3 * tcs; i += blockDim.x) {
-                const int c = i / tcs, rr = i - c * tcs;
-                const int iy = rr / tx, ix = rr - iy * tx;
-                tile[i] = u[c * G.cs + (size_t)(G.g - R + iy) * G.nx + (G.g - R + ix)];
-            }
-        }
-        __syncthreads();
-    }
-    (void)ty;
+    const int tx = G.bs0 + 2 * R, tcs = tx * (ty0 + 2 * R), cs = (int)G.cs;
+    const int npts = G.bs0 * ty0, nall = G.bs0 * G.bs1, nt = (int)blockDim.x, tid = (int)threadIdx.x;
+    const double *u = in + (size_t)b * G.blk;
+    const StageBlk SB = FUSED ? stage_blk<3>(sa, b, G.blk, nall) : StageBlk{};
     const double dx0 = x0dx[6 * k + 3], dx1 = x0dx[6 * k + 4];
+    // what to add to a place in the ghost nodes beyond face f to read it there
+    auto face = [&](int f) -> ptrdiff_t {
+        const int nb = faces ? faces[f] : -1;
+        const int sh = f < 2 ? G.bs0 : G.bs1 * G.nx;
+        return nb < 0 ? 0 : ((ptrdiff_t)nb - b) * (ptrdiff_t)G.blk + (f & 1 ? -sh : sh);
+    };
+    const ptrdiff_t fxm = face(0), fxp = face(1), fym = y0 == 0 ? face(2) : 0,
+                    fyp = y0 + ty0 == G.bs1 ? face(3) : 0;
+    // halo position h of the slab: its place in the tile and where it is read
+    const int nrow = 2 * R * G.bs0, nhalo = nrow + 2 * R * ty0;
+    auto halo = [&](int h, int &l) -> const double * {
+        int px, py;
+        ptrdiff_t o;
+        if (h < nrow) {  // rows below and above
+            const int r = h / G.bs0;
+            px = R + h - r * G.bs0;
+            py = r < R ? r : ty0 + r;
+            o = r < R ? fym : fyp;
+        } else {  // columns left and right
+            const int e = h - nrow, r = e / (2 * R), c = e - r * (2 * R);
+            py = R + r;
+            px = c < R ? c : G.bs0 + c;
+            o = c < R ? fxm : fxp;
+        }
+        l = py * tx + px;
+        return u + o + (ptrdiff_t)(G.g + y0 - R + py) * G.nx + (G.g - R + px);
+    };
+    const int iy0 = tid / G.bs0, ix0 = tid - iy0 * G.bs0;
+    const int gi0 = (G.g + y0 + iy0) * G.nx + G.g + ix0;
+    MaskReg mpre{};
+    mpre.has = mk != nullptr;
+    double upt[3] = {0, 0, 0}, hv[3] = {0, 0, 0}, apre[3] = {0, 0, 0}, upre[3] = {0, 0, 0};
+    int hl = 0;
+    if (tid < npts) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) upt[c] = u[c * cs + gi0];
+    }
+    if (tid < nhalo) {
+        const double *h = halo(tid, hl);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) hv[c] = h[c * cs];
+    }
+    if (tid < npts) {
+        if (mk) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c)
+                if (c != 3) mpre.v[c] = mk[c * cs + gi0];  // component 3 (u_s,z) is 3D only
+        }
+        if (FUSED && sa.mode >= 1) {
+            const int p = y0 * G.bs0 + tid;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) apre[c] = SB.acc[c * nall + p];
+            if (sa.mode == 1) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) upre[c] = SB.u0[c * cs + gi0];
+            }
+        }
+    }
     const double inv[2] = {1.0 / dx0, 1.0 / dx1};
     const double inv2[2] = {1.0 / (dx0 * dx0), 1.0 / (dx1 * dx1)};
-    for (int pnt = threadIdx.x; pnt < npts; pnt += blockDim.x) {
-        const int iy = pnt / G.bs0, ix = pnt - iy * G.bs0;
+    if (tid < npts) {
+        double *t = tile + (iy0 + R) * tx + ix0 + R;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) t[c * tcs] = upt[c];
+    }
+    if (tid < nhalo) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) tile[c * tcs + hl] = hv[c];
+    }
+    for (int p = tid + nt; p < npts; p += nt) {  // slabs with more points or halo than threads
+        const int iy = p / G.bs0, ix = p - iy * G.bs0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            tile[c * tcs + (iy + R) * tx + ix + R] = u[c * cs + (G.g + y0 + iy) * G.nx + G.g + ix];
+    }
+    for (int h = tid + nt; h < nhalo; h += nt) {
+        int l;
+        const double *src = halo(h, l);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) tile[c * tcs + l] = src[c * cs];
+    }
+    __syncthreads();
+    auto point = [&](int iy, int ix, const auto &m, auto &&epilogue) {
         const double *uc = tile + (iy + R) * tx + (ix + R);
-        const int gi = (G.g + iy) * G.nx + (G.g + ix);
+        const int gi = (G.g + y0 + iy) * G.nx + (G.g + ix);
         double r[3];
         const StridedAcc<2> A{uc, tcs, {1, tx, 0}};
-        if (PRE && pnt == p0) {
-            // separate calls (not a pointer select) keep mpre in registers
-            if (mk) acm_point<2, S, SKEW>(A, inv, inv2, a, mpre, 1, r);
-            else acm_point<2, S, SKEW>(A, inv, inv2, a, nullptr, 1, r);
-            if constexpr (FUSED) stage_epilogue_pre<3>(sa, SB, k, gi, cs, pnt, npts, r, uc, tcs, apre, upre);
+        acm_point<2, S, SKEW>(A, inv, inv2, a, m, r);
+        if constexpr (FUSED) {
+            epilogue(gi, (y0 + iy) * G.bs0 + ix, r, uc);
         } else {
-            acm_point<2, S, SKEW>(A, inv, inv2, a, mk ? mk + gi : nullptr, G.cs, r);
-            if constexpr (FUSED) stage_epilogue<3>(sa, SB, k, gi, cs, pnt, npts, r, uc, tcs);
-        }
-        if constexpr (!FUSED) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) out[base + gi + c * G.cs] = r[c];
+            for (int c = 0; c < 3; ++c) out[(size_t)b * G.blk + gi + c * cs] = r[c];
         }
+    };
+    if (tid < npts)
+        point(iy0, ix0, mpre, [&](int gi, int p, const double *r, const double *uc) {
+            stage_epilogue_pre<3>(sa, SB, k, gi, cs, p, nall, r, uc, tcs, apre, upre);
+        });
+    for (int pnt = tid + nt; pnt < npts; pnt += nt) {
+        const int iy = pnt / G.bs0, ix = pnt - iy * G.bs0;
+        const int gi0n = (G.g + y0 + iy) * G.nx + (G.g + ix);
+        point(iy, ix, MaskMem{mk ? mk + gi0n : nullptr, cs}, [&](int gi, int p, const double *r, const double *uc) {
+            stage_epilogue<3>(sa, SB, k, gi, cs, p, nall, r, uc, tcs);
+        });
     }
-    if constexpr (FUSED) stage_ghost_cols_2d<3>(sa, SB, G);
+    if constexpr (FUSED) stage_ghost_cols_2d<3>(sa, SB, G, y0, ty0);
 }
 
-template <int S, bool SKEW, bool FUSED, bool PRE>
+template <int S, bool SKEW, bool FUSED>
 __global__ __launch_bounds__(256) void k_rhs2d(const double *__restrict__ in, double *__restrict__ out,
                                                const double *__restrict__ mask,
                                                const int32_t *__restrict__ act,
                                                const double *__restrict__ x0dx, Geo G, AcmDev a,
-                                               StageArgs sa)
+                                               StageArgs sa, int ysplit, int ty0)
 {
     extern __shared__ double tile[];
-    const int k = blockIdx.x;
+    const int wg = xcd_swizzle((int)blockIdx.x, (int)gridDim.x);
+    const int k = wg / ysplit, y0 = (wg - k * ysplit) * ty0;
     const int b = act[k];
     const double *mk = mask ? mask + (G.mask_per_block ? (size_t)b * G.mblk : 0) : nullptr;
-    rhs2d_block<S, SKEW, FUSED, PRE>(tile, in, out, mk, b, k, x0dx, G, a, sa);
+    rhs2d_slab<S, SKEW, FUSED>(tile, in, out, mk, b, k, y0, min(ty0, G.bs1 - y0), x0dx,
+                               FUSED && sa.gnb ? sa.gnb + (size_t)k * 4 : nullptr, G, a, sa);
 }
 
 // ---------------------------------------------------------------------------
 // Several pools in one launch (independent forests of a batch, any block
-// size): entry k of the launch is position k - ent0 of the active list of
-// the pool whose entry range holds k (pools[] in entry order), with that
+// size): item k of the launch is a part (2D: one of nslab slabs, 3D: the
+// whole) of the block at position (k - ent0) / nslab of the active list of
+// the pool whose item range holds k (pools[] in item order), with that
 // position's origin/spacing and block group g = goff + grp[..] (dt dtg[g],
 // constants gacm[g]), all read from the pool's own device tables; once per
-// step k_entries resolves every entry into a record (pool, hvy id, group,
-// position) that the stage kernels read with one load per block.  The
+// step k_entries resolves every item into a record (MEnt) that the stage
+// kernels read with one load.  The
 // stage's input and output arrays are selected per pool from arr[]:
 // 0 hvy_block, 1 work slot 0 (the RK accumulator), 2 / 3 work slots 1 / 2.
-// The kernels are persistent (grid-stride over the entries, their count read
+// The kernels are persistent (grid-stride over the items, their count read
 // from device memory), so one captured launch serves any number of blocks.
 // ---------------------------------------------------------------------------
 // the last pool whose first entry (s < 0), first chunk of sync stage s (0..2) or
@@ -505,7 +512,7 @@ __device__ __forceinline__ StageArgs multi_stage_args(const MPoolDev &P, const M
     return sa;
 }
 
-// the entry records of a launch: one thread per entry
+// the item records of a launch: one thread per item
 __global__ __launch_bounds__(256) void k_entries(const MPoolDev *__restrict__ pools, int npools,
                                                  const int64_t *__restrict__ tot, MEnt *__restrict__ ents)
 {
@@ -513,207 +520,46 @@ __global__ __launch_bounds__(256) void k_entries(const MPoolDev *__restrict__ po
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         const int p = pool_of(pools, npools, k, -1);
         const MPoolDev &P = pools[p];
-        const int j = k - P.ent0;
-        ents[k] = MEnt{p, P.act[j], P.goff + P.grp[j], j};
+        const int j = (k - P.ent0) / P.nslab, y0 = (k - P.ent0 - j * P.nslab) * P.ty0;
+        ents[k] = MEnt{p, P.act[j], P.goff + P.grp[j], j, y0, min(P.ty0, P.G.bs1 - y0)};
     }
 }
 
-// entry k's record with every field wave-uniform, so that the descriptor and
+// an item's record with every field wave-uniform, so that the descriptor and
 // the group's constants are read through scalar loads
-__device__ __forceinline__ MEnt entry_of(const MEnt *__restrict__ ents, int k)
+__device__ __forceinline__ MEnt uniform(const MEnt &e)
 {
-    const MEnt e = ents[k];
     return MEnt{__builtin_amdgcn_readfirstlane(e.pool), __builtin_amdgcn_readfirstlane(e.b),
-                __builtin_amdgcn_readfirstlane(e.g), __builtin_amdgcn_readfirstlane(e.j)};
+                __builtin_amdgcn_readfirstlane(e.g),    __builtin_amdgcn_readfirstlane(e.j),
+                __builtin_amdgcn_readfirstlane(e.y0),   __builtin_amdgcn_readfirstlane(e.ty0)};
 }
 
-// PRE: the first point's mask and operands loaded before the tile barrier;
-// WPE: minimum waves per SIMD the register allocation must allow.
-template <int S, bool SKEW, bool PRE, int WPE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void k_rhs2d_multi(
-    const MPoolDev *__restrict__ pools, const MEnt *__restrict__ ents, const double *__restrict__ dtg,
-    const AcmDev *__restrict__ gacm, const int64_t *__restrict__ tot, MStage st)
+// 2D: items are slabs (slab_rows) of the pools' blocks; the next item's record
+// is requested while an item is worked on.
+template <int S, bool SKEW>
+__global__ __launch_bounds__(256) void k_rhs2d_multi(const MPoolDev *__restrict__ pools,
+                                                     const MEnt *__restrict__ ents, const double *__restrict__ dtg,
+                                                     const AcmDev *__restrict__ gacm,
+                                                     const int64_t *__restrict__ tot, MStage st)
 {
     extern __shared__ double tile[];
     const int nent = (int)tot[0];
-    for (int k = blockIdx.x; k < nent; k += gridDim.x) {
-        const MEnt e = entry_of(ents, k);
+    int k = blockIdx.x;
+    if (k >= nent) return;
+    MEnt next = ents[k];
+    for (; k < nent; k += gridDim.x) {
+        const MEnt e = uniform(next);
+        next = ents[min(k + (int)gridDim.x, nent - 1)];
         const MPoolDev &P = pools[e.pool];
-        const int j = e.j, b = e.b, g = e.g;
+        const int b = e.b, g = e.g;
         const Geo &G = P.G;
         const AcmDev &a = gacm[g];
         const StageArgs sa = multi_stage_args(P, st, dtg + g);
         const double *mk = P.mask ? P.mask + (G.mask_per_block ? (size_t)b * G.mblk : 0) : nullptr;
-        rhs2d_block<S, SKEW, true, PRE>(tile, P.arr[st.in_sel], nullptr, mk, b, 0, P.x0dx + 6 * (size_t)j, G, a,
-                                        sa);
-        __syncthreads();  // the tile is reused by the next entry
+        rhs2d_slab<S, SKEW, true>(tile, P.arr[st.in_sel], nullptr, mk, b, 0, e.y0, e.ty0, P.x0dx + 6 * (size_t)e.j,
+                                  nullptr, G, a, sa);
+        __syncthreads();  // the tile is reused by the next item
     }
-}
-
-// 2D, several pools, software-pipelined: while block k is computed from
-// the LDS tile, the workgroup already holds the next entry's metadata and
-// has its halo tile in flight into registers; after the compute the
-// registers go to LDS.  The tile is loaded by rows: lane (col, row0) =
-// (t % 32, t / 32) takes column col of rows row0, row0 + 8, ... of every
-// component, so a wavefront reads two contiguous row segments and no index
-// is divided.  Needs tile widths <= 32 and heights <= 8 * MP_ROWS (Bs up to
-// 28 with FD4); per block the arithmetic is that of k_rhs2d_multi.
-constexpr int MP_ROWS = 4;
-template <int S, bool SKEW>
-__global__ __launch_bounds__(256) void k_rhs2d_multi_pipe(const MPoolDev *__restrict__ pools,
-                                                          const MEnt *__restrict__ ents,
-                                                          const double *__restrict__ dtg,
-                                                          const AcmDev *__restrict__ gacm,
-                                                          const int64_t *__restrict__ tot, MStage st)
-{
-    constexpr int R = Reach<S>::R;
-    extern __shared__ double tile[];
-    const int nent = (int)tot[0];
-    int k = blockIdx.x;
-    if (k >= nent) return;  // uniform over the workgroup
-    const int col = threadIdx.x & 31, row0 = threadIdx.x >> 5;
-    double reg[3][MP_ROWS];
-    int cp, cj, cb, cg;  // the current entry: pool, active position, hvy id, group
-    auto fetch = [&](int kk, int &p, int &j, int &b, int &g) {
-        const MEnt e = entry_of(ents, kk);
-        p = e.pool;
-        j = e.j;
-        b = e.b;
-        g = e.g;
-        const MPoolDev &P = pools[p];
-        const Geo &G = P.G;
-        const int tx = G.bs0 + 2 * R, ty = G.bs1 + 2 * R;
-        const double *u = P.arr[st.in_sel] + (size_t)b * G.blk + (size_t)(G.g - R) * G.nx + (G.g - R);
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-#pragma unroll
-            for (int r = 0; r < MP_ROWS; ++r) {
-                const int row = row0 + 8 * r;
-                if (col < tx && row < ty) reg[c][r] = u[c * G.cs + (size_t)row * G.nx + col];
-            }
-    };
-    fetch(k, cp, cj, cb, cg);
-    while (true) {
-        __syncthreads();  // the previous block is done with the tile
-        {
-            const Geo &G = pools[cp].G;
-            const int tx = G.bs0 + 2 * R, ty = G.bs1 + 2 * R, tcs = tx * ty;
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-#pragma unroll
-                for (int r = 0; r < MP_ROWS; ++r) {
-                    const int row = row0 + 8 * r;
-                    if (col < tx && row < ty) tile[c * tcs + row * tx + col] = reg[c][r];
-                }
-        }
-        __syncthreads();
-        const int kn = k + (int)gridDim.x;
-        int np = 0, nj = 0, nb = 0, ng = 0;
-        if (kn < nent) fetch(kn, np, nj, nb, ng);  // in flight while block k is computed
-        const MPoolDev &P = pools[cp];
-        const Geo G = P.G;
-        const AcmDev a = gacm[cg];
-        const StageArgs sa = multi_stage_args(P, st, dtg + cg);
-        const double *mk = P.mask ? P.mask + (G.mask_per_block ? (size_t)cb * G.mblk : 0) : nullptr;
-        rhs2d_block<S, SKEW, true, false, true>(tile, nullptr, nullptr, mk, cb, 0, P.x0dx + 6 * (size_t)cj, G, a, sa);
-        if (kn >= nent) break;  // uniform
-        k = kn;
-        cp = np;
-        cj = nj;
-        cb = nb;
-        cg = ng;
-    }
-}
-
-// 2D, persistent and software-pipelined: workgroup w handles the blocks at
-// active positions w, w + G, w + 2G, ... (G workgroups); the halo tile of its
-// next block is loaded into registers while the current block is computed
-// from LDS, then stored to the other of two LDS buffers.  Per point the
-// arithmetic is that of k_rhs2d.
-constexpr int PIPE_MAXL = 6;  // tile elements per thread held in registers
-template <int S, bool SKEW, bool FUSED>
-__global__ __launch_bounds__(256) void k_rhs2d_pipe(const double *__restrict__ in, double *__restrict__ out,
-                                                    const double *__restrict__ mask,
-                                                    const int32_t *__restrict__ act,
-                                                    const double *__restrict__ x0dx, Geo G, AcmDev a,
-                                                    StageArgs sa, int nact)
-{
-    constexpr int R = Reach<S>::R;
-    extern __shared__ double sm[];
-    const int tx = G.bs0 + 2 * R, ty = G.bs1 + 2 * R, tcs = tx * ty, ntile = 3 * tcs;
-    const int npts = G.bs0 * G.bs1;
-    double reg[PIPE_MAXL];
-    int off[PIPE_MAXL];  // block-independent source offsets of this thread's tile elements
-#pragma unroll
-    for (int j = 0; j < PIPE_MAXL; ++j) {
-        const int i = threadIdx.x + j * blockDim.x;
-        const int c = i / tcs, rr = i - c * tcs;
-        const int iy = rr / tx, ix = rr - iy * tx;
-        off[j] = i < ntile ? (int)(c * G.cs + (size_t)(G.g - R + iy) * G.nx + (G.g - R + ix)) : 0;
-    }
-    int k = blockIdx.x;
-    if (k >= nact) return;  // uniform over the workgroup
-    auto load = [&](int kk) {
-        const double *u = in + (size_t)act[kk] * G.blk;
-#pragma unroll
-        for (int j = 0; j < PIPE_MAXL; ++j)
-            if (threadIdx.x + j * blockDim.x < (unsigned)ntile) reg[j] = u[off[j]];
-    };
-    auto store = [&](double *dst) {
-#pragma unroll
-        for (int j = 0; j < PIPE_MAXL; ++j) {
-            const int i = threadIdx.x + j * blockDim.x;
-            if (i < ntile) dst[i] = reg[j];
-        }
-    };
-    load(k);
-    store(sm);
-    __syncthreads();
-    int cur = 0;
-    while (true) {
-        const int kn = k + (int)gridDim.x;
-        if (kn < nact) load(kn);  // in flight while block k is computed
-        const double *tile = sm + cur * ntile;
-        const int b = act[k];
-        const double dx0 = x0dx[6 * k + 3], dx1 = x0dx[6 * k + 4];
-        const double inv[2] = {1.0 / dx0, 1.0 / dx1};
-        const double inv2[2] = {1.0 / (dx0 * dx0), 1.0 / (dx1 * dx1)};
-        const double *mk = mask ? mask + (G.mask_per_block ? (size_t)b * G.mblk : 0) : nullptr;
-        for (int pnt = threadIdx.x; pnt < npts; pnt += blockDim.x) {
-            const int iy = pnt / G.bs0, ix = pnt - iy * G.bs0;
-            const double *uc = tile + (iy + R) * tx + (ix + R);
-            const size_t gi = (size_t)(G.g + iy) * G.nx + (G.g + ix);
-            double r[3];
-            const StridedAcc<2> A{uc, tcs, {1, tx, 0}};
-            acm_point<2, S, SKEW>(A, inv, inv2, a, mk ? mk + gi : nullptr, G.cs, r);
-            const size_t o = (size_t)b * G.blk + gi;
-            if constexpr (FUSED) {
-                const StageBlk SB = stage_blk<3>(sa, b, G.blk, npts);
-                stage_epilogue<3>(sa, SB, k, (int)gi, (int)G.cs, pnt, npts, r, uc, tcs);
-            } else {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) out[o + c * G.cs] = r[c];
-            }
-        }
-        if constexpr (FUSED) stage_ghost_cols_2d<3>(sa, stage_blk<3>(sa, b, G.blk, npts), G);
-        if (kn >= nact) break;  // uniform
-        store(sm + (cur ^ 1) * ntile);
-        __syncthreads();
-        cur ^= 1;
-        k = kn;
-    }
-}
-
-// Workgroups are dispatched to the 8 XCDs (each with its own L2) round-robin:
-// workgroup w runs on XCD w % 8.  The swizzle gives XCD x the consecutive
-// logical indices [start(x), start(x) + count(x)), so the workgroups of one
-// block share an L2 instead of being spread over all eight.  A permutation
-// of [0, nw) for any nw.
-__device__ __forceinline__ int xcd_swizzle(int w, int nw)
-{
-    constexpr int NX = 8;
-    const int q = nw / NX, r = nw - q * NX, x = w % NX;
-    return x * q + min(x, r) + w / NX;
 }
 
 // 3D: 256 interior points per workgroup, stencil reads served by L1/L2;
@@ -741,7 +587,7 @@ __global__ __launch_bounds__(256) void k_rhs3d(const double *__restrict__ in, do
     const double *mk = mask ? mask + (G.mask_per_block ? (size_t)b * G.mblk : 0) + gi : nullptr;
     double r[4];
     const StridedAcc<3> A{uc, (ptrdiff_t)G.cs, {1, G.nx, (ptrdiff_t)G.nx * G.ny}};
-    acm_point<3, S, SKEW>(A, inv, inv2, a, mk, G.cs, r);
+    acm_point<3, S, SKEW>(A, inv, inv2, a, MaskMem{mk, (ptrdiff_t)G.cs}, r);
     const size_t o = (size_t)b * G.blk + gi;
     if constexpr (FUSED) {
         const StageBlk SB = stage_blk<4>(sa, b, G.blk, npts);
@@ -771,7 +617,7 @@ __global__ __launch_bounds__(256) void k_rhs3d_multi(const MPoolDev *__restrict_
         const int w = XCD ? xcd_swizzle(t, total) : t;
         const int k = w / nchunk;
         const int pnt = (w - k * nchunk) * 256 + threadIdx.x;
-        const MEnt e = entry_of(ents, k);
+        const MEnt e = uniform(ents[k]);
         const MPoolDev &P = pools[e.pool];
         const Geo &G = P.G;
         const int npts = G.bs0 * G.bs1 * G.bs2;
@@ -789,7 +635,7 @@ __global__ __launch_bounds__(256) void k_rhs3d_multi(const MPoolDev *__restrict_
         const double *mk = P.mask ? P.mask + (G.mask_per_block ? (size_t)b * G.mblk : 0) + gi : nullptr;
         double r[4];
         const StridedAcc<3> A{uc, (ptrdiff_t)G.cs, {1, G.nx, (ptrdiff_t)G.nx * G.ny}};
-        acm_point<3, S, SKEW>(A, inv, inv2, a, mk, G.cs, r);
+        acm_point<3, S, SKEW>(A, inv, inv2, a, MaskMem{mk, (ptrdiff_t)G.cs}, r);
         const StageBlk SB = stage_blk<4>(sa, b, G.blk, npts);
         stage_epilogue<4>(sa, SB, 0, (int)gi, (int)G.cs, pnt, npts, r, uc, G.cs);
         stage_ghost_cols<4>(sa, SB, (int)gi - (G.g + ix), (int)G.cs, ix, G.bs0, G.g);
@@ -938,7 +784,7 @@ __global__ __launch_bounds__(512) void k_rhs3d_zm(const double *__restrict__ in,
             return plane[c * tcs + lc + o * (d == 0 ? 1 : tx)];
         };
         double r[4];
-        acm_point<3, S, SKEW>(A, inv, inv2, a, mk ? mk + gi : nullptr, G.cs, r);
+        acm_point<3, S, SKEW>(A, inv, inv2, a, MaskMem{mk ? mk + gi : nullptr, (ptrdiff_t)G.cs}, r);
         if constexpr (FUSED) {
             const double u0c[4] = {q[0][R], q[1][R], q[2][R], q[3][R]};
             stage_epilogue_pre<4>(sa, SB, k, gi, cs, pnt, npts, r, u0c, 1, apre, upre);
@@ -977,6 +823,24 @@ bool zm_valid(int bs0, int bs1, int scheme, int ys)
     if (nthr < 64 || nthr > 512) return false;
     if (2 * R * (bs0 + ty0) > nthr) return false;
     return sizeof(double) * 4 * (bs0 + 2 * R) * (ty0 + 2 * R) <= 64 * 1024;
+}
+
+// the 2D stages take blocks whose whole tile would fit a compute unit's LDS
+bool tile2d_ok(int bs0, int bs1, int R)
+{
+    return sizeof(double) * 3 * (bs0 + 2 * R) * (bs1 + 2 * R) <= 160 * 1024;
+}
+
+// Rows of a 2D slab: as many as give at most 256 points, a thread each, and
+// slabs of about equal size.  Launch times of a fused FD4 stage by the number
+// of slabs a block is cut into: 64 blocks of 32^2 (skew-symmetric) 9.6 / 6.1 /
+// 4.3 / 4.7 us in 1 / 2 / 4 / 6, 4096 of 24^2 46 / 47 / 39 / 44 us in 1 / 2 /
+// 3 / 4, 1024 of 48^2 58 / 45 / 41 / 39 us in 1 / 2 / 4 / 6; 16^2 whole 4.3 us
+// for 256 blocks, in 2 slabs 4.6.
+int slab_rows(int bs0, int bs1)
+{
+    const int most = std::max(1, 256 / bs0), ys = (bs1 + most - 1) / most;
+    return (bs1 + ys - 1) / ys;
 }
 
 // y-split of the 3D stage kernel: the pool's tuned value, or of the valid
@@ -1050,45 +914,14 @@ static int dispatch_rhs(wh_pool *P, const AcmDev &a, const double *in, double *o
     const Geo G = make_geo(P);
     const double *mask = (P->mask && (a.penal || a.sponge)) ? P->mask : nullptr;
     if (P->d.dim == 2) {
-        int R = a.scheme == WH_FD2 ? 1 : a.scheme == WH_FD4 ? 2 : 3;
-        size_t lds = sizeof(double) * 3 * (G.bs0 + 2 * R) * (G.bs1 + 2 * R);
-        WH_CHECK(lds <= 160 * 1024, WH_E_ARG, "2D block tile exceeds LDS");
-        const int pre = P->k2d_stage == 1;
-        // the persistent pipelined variant: two tiles in LDS, each thread
-        // holds at most PIPE_MAXL tile elements of the next block
-        // (the halo gather reads through the one-workgroup-per-block kernel)
-        const int wpc = (FUSED && sa.gnb) ? 0 : P->k2d_stage == 2 ? 2 : P->k2d_stage == 3 ? 4 : P->k2d_stage == 4 ? 8 : 0;
-        if (wpc && 3 * (G.bs0 + 2 * R) * (G.bs1 + 2 * R) <= PIPE_MAXL * 256 && 2 * lds <= 160 * 1024) {
-            const int nwg = std::min(nact, wpc * P->n_cu);
-            dim3 pgrid(nwg), pblock(256);
-#define L2P(SC, SK)                                                                                 \
-    hipLaunchKernelGGL((k_rhs2d_pipe<SC, SK, FUSED>), pgrid, pblock, 2 * lds, P->stream, in, out, mask, \
-                       act, x0dx, G, a, sa, nact)
-            switch (a.scheme * 2 + a.skew) {
-            case WH_FD2 * 2: L2P(WH_FD2, false); break;
-            case WH_FD2 * 2 + 1: L2P(WH_FD2, true); break;
-            case WH_FD4 * 2: L2P(WH_FD4, false); break;
-            case WH_FD4 * 2 + 1: L2P(WH_FD4, true); break;
-            case WH_FD4_TW * 2: L2P(WH_FD4_TW, false); break;
-            case WH_FD4_TW * 2 + 1: L2P(WH_FD4_TW, true); break;
-            case WH_FD6 * 2: L2P(WH_FD6, false); break;
-            case WH_FD6 * 2 + 1: L2P(WH_FD6, true); break;
-            default: set_error("unknown scheme"); return WH_E_ARG;
-            }
-#undef L2P
-            WH_HIP(hipGetLastError());
-            return WH_OK;
-        }
-        dim3 grid(nact), blockd(256);
-#define L2D(SC, SK)                                                                              \
-    do {                                                                                         \
-        if (pre)                                                                                 \
-            hipLaunchKernelGGL((k_rhs2d<SC, SK, FUSED, true>), grid, blockd, lds, P->stream, in, out, \
-                               mask, act, x0dx, G, a, sa);                                       \
-        else                                                                                     \
-            hipLaunchKernelGGL((k_rhs2d<SC, SK, FUSED, false>), grid, blockd, lds, P->stream, in,     \
-                               out, mask, act, x0dx, G, a, sa);                                  \
-    } while (0)
+        const int R = reach_of(a.scheme);
+        const int ty0 = slab_rows(G.bs0, G.bs1), ys = (G.bs1 + ty0 - 1) / ty0;
+        const size_t lds = sizeof(double) * 3 * (G.bs0 + 2 * R) * (ty0 + 2 * R);
+        WH_CHECK(tile2d_ok(G.bs0, G.bs1, R), WH_E_ARG, "2D block tile exceeds LDS");
+        const dim3 grid(nact * ys), blockd(std::min(256, (G.bs0 * ty0 + 63) / 64 * 64));
+#define L2D(SC, SK)                                                                                             \
+    hipLaunchKernelGGL((k_rhs2d<SC, SK, FUSED>), grid, blockd, lds, P->stream, in, out, mask, act, x0dx, G, a, sa, \
+                       ys, ty0)
         switch (a.scheme * 2 + a.skew) {
         case WH_FD2 * 2: L2D(WH_FD2, false); break;
         case WH_FD2 * 2 + 1: L2D(WH_FD2, true); break;
@@ -1378,29 +1211,13 @@ int launch_entries(hipStream_t stream, const MPoolDev *d_pools, int npools, cons
 
 int launch_stage_multi(hipStream_t stream, int dim, int scheme, int skew, int xcd, const MPoolDev *d_pools,
                        int npools, const MEnt *d_ents, const double *d_dtg, const AcmDev *d_gacm,
-                       const int64_t *d_tot, const MStage &ms, size_t lds, int grid, int nchunk, int pipe)
+                       const int64_t *d_tot, const MStage &ms, size_t lds, int grid, int nchunk)
 {
     (void)npools;
     if (dim == 2) {
-        WH_CHECK(lds <= 160 * 1024, WH_E_ARG, "2D block tile exceeds LDS");
-#define M2D(SC, SK)                                                                                              \
-    do {                                                                                                         \
-        if (pipe == 1)                                                                                           \
-            hipLaunchKernelGGL((k_rhs2d_multi_pipe<SC, SK>), dim3(grid), dim3(256), lds, stream, d_pools, d_ents, \
-                               d_dtg, d_gacm, d_tot, ms);                                                        \
-        else if (pipe == 2)                                                                                      \
-            hipLaunchKernelGGL((k_rhs2d_multi<SC, SK, false, 1>), dim3(grid), dim3(256), lds, stream, d_pools,    \
-                               d_ents, d_dtg, d_gacm, d_tot, ms);                                                \
-        else if (pipe == 3)                                                                                      \
-            hipLaunchKernelGGL((k_rhs2d_multi<SC, SK, false, 6>), dim3(grid), dim3(256), lds, stream, d_pools,    \
-                               d_ents, d_dtg, d_gacm, d_tot, ms);                                                \
-        else if (pipe == 4)                                                                                      \
-            hipLaunchKernelGGL((k_rhs2d_multi<SC, SK, false, 8>), dim3(grid), dim3(256), lds, stream, d_pools,    \
-                               d_ents, d_dtg, d_gacm, d_tot, ms);                                                \
-        else                                                                                                     \
-            hipLaunchKernelGGL((k_rhs2d_multi<SC, SK, true, 1>), dim3(grid), dim3(256), lds, stream, d_pools,     \
-                               d_ents, d_dtg, d_gacm, d_tot, ms);                                                \
-    } while (0)
+#define M2D(SC, SK)                                                                                           \
+    hipLaunchKernelGGL((k_rhs2d_multi<SC, SK>), dim3(grid), dim3(256), lds, stream, d_pools, d_ents, d_dtg, d_gacm, \
+                       d_tot, ms)
         switch (scheme * 2 + skew) {
         case WH_FD2 * 2: M2D(WH_FD2, false); break;
         case WH_FD2 * 2 + 1: M2D(WH_FD2, true); break;
