@@ -348,8 +348,7 @@ __device__ __forceinline__ void rhs2d_slab(double *tile, const double *__restric
         const int sh = f < 2 ? G.bs0 : G.bs1 * G.nx;
         return nb < 0 ? 0 : ((ptrdiff_t)nb - b) * (ptrdiff_t)G.blk + (f & 1 ? -sh : sh);
     };
-    const ptrdiff_t fxm = face(0), fxp = face(1), fym = y0 == 0 ? face(2) : 0,
-                    fyp = y0 + ty0 == G.bs1 ? face(3) : 0;
+    const ptrdiff_t fxm = face(0), fxp = face(1), fym = face(2), fyp = face(3);
     // halo position h of the slab: its place in the tile and where it is read
     const int nrow = 2 * R * G.bs0, nhalo = nrow + 2 * R * ty0;
     auto halo = [&](int h, int &l) -> const double * {
@@ -359,7 +358,8 @@ __device__ __forceinline__ void rhs2d_slab(double *tile, const double *__restric
             const int r = h / G.bs0;
             px = R + h - r * G.bs0;
             py = r < R ? r : ty0 + r;
-            o = r < R ? fym : fyp;
+            const int y = y0 - R + py;  // a slab of fewer than R rows reaches beyond the face from inside, too
+            o = y < 0 ? fym : y >= G.bs1 ? fyp : 0;
         } else {  // columns left and right
             const int e = h - nrow, r = e / (2 * R), c = e - r * (2 * R);
             py = R + r;
