@@ -569,6 +569,7 @@ int wh_pool_create(wh_pool **out, const wh_pool_desc *desc)
         return fail("hipHostMalloc", e);
     if ((e = hipMemsetAsync(P->scal, 0, sizeof(double) * DS_COUNT, P->stream)) != hipSuccess)
         return fail("hipMemset", e);
+    if (launch_set_scalar(P, DS_DTACC, DT_NONE) != WH_OK) return fail("scalars", hipErrorUnknown);
     if ((e = hipMemsetAsync(P->block, 0, sizeof(double) * P->blk * d.nb_max, P->stream)) != hipSuccess)
         return fail("hipMemset", e);
     if (P->work && (e = hipMemsetAsync(P->work, 0, sizeof(double) * P->blk * d.nb_max * d.n_work_slots,
@@ -1028,10 +1029,7 @@ int wh_rk_step_groups(wh_pool *P, const wh_acm_params *p, const double *bt, int 
 int wh_time_set(wh_pool *P, double time, int iteration)
 {
     WH_CHECK(P, WH_E_ARG, "null argument");
-    int rc = launch_set_scalar(P, DS_TIME, time);
-    if (!rc) rc = launch_set_scalar(P, DS_ITER, (double)iteration);
-    if (!rc) rc = launch_set_scalar(P, DS_DT, 0.0);
-    if (rc) return rc;
+    if (int rc = launch_time_set(P, time, (double)iteration)) return rc;
     WH_HIP(hipStreamSynchronize(P->stream));
     return WH_OK;
 }
@@ -1071,11 +1069,8 @@ int wh_time_fetched(wh_pool *P, double *time, int *iteration, double *dt_last)
 static int one_device_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
                            const TimeDev &tc)
 {
-    int rc;
-    if ((rc = launch_dt(P, a))) return rc;
-    if ((rc = launch_dt_finalize(P, tc))) return rc;
-    if ((rc = fused_step(P, a, bt, nrows))) return rc;
-    return launch_time_advance(P);
+    if (int rc = launch_dt(P, a, &tc)) return rc;
+    return fused_step(P, a, bt, nrows);
 }
 
 int wh_run_steps(wh_pool *P, const wh_acm_params *p, const double *bt, int nrows,

@@ -38,8 +38,13 @@ enum DevScalar {
     DS_TIME = 2,         // current time (device-side time loop)
     DS_DT = 3,           // dt of the current step
     DS_ITER = 4,         // iteration counter (stored as double)
+    DS_DTACC = 5,        // uint64 bits: the running minimum of a dt launch, DT_NONE between launches
+    DS_DTCNT = 6,        // uint64: the workgroups of it that are done, 0 between launches
     DS_COUNT = 8
 };
+
+// the minimum block dt over no blocks (calculate_time_step.f90:28)
+constexpr double DT_NONE = 9.0e9;
 
 // Kernel-side copy of the ACM parameters.
 struct AcmDev {
@@ -266,7 +271,9 @@ int launch_sync(wh_pool *P, int sync_case, double *arr, int one_receiver);
 int launch_combine(wh_pool *P, double *out, const double *base, int nterms,
                    const double *const *terms, const double *coefs, const int32_t *act,
                    int nact);
-int launch_dt(wh_pool *P, const AcmDev &a);
+// the minimum block dt into DS_DTMIN_BITS; with step also its clamps into
+// DS_DT and the time advance of the step that follows
+int launch_dt(wh_pool *P, const AcmDev &a, const TimeDev *step = nullptr);
 int launch_maxabs(wh_pool *P, const double *in);
 // dtb: per active-list position dt (block groups), or null for the pool's DS_DT
 // gnb: the face table (FaceGather; 3D: of the z-marching kernel), or null
@@ -277,8 +284,7 @@ int launch_fused_stage(wh_pool *P, const AcmDev &a, const double *tin, double *t
 int launch_dt_groups(wh_pool *P, const AcmDev &a);
 // whether the 3D stages run the z-marching kernel (the one that can gather)
 bool stage_gathers(const wh_pool *P, int scheme);
-int launch_dt_finalize(wh_pool *P, const TimeDev &tc);
-int launch_time_advance(wh_pool *P);
+int launch_time_set(wh_pool *P, double time, double iter);
 int launch_set_scalar(wh_pool *P, int which, double v);
 
 // the chunks of patch i of a list (its points cut into pieces of

@@ -1685,71 +1685,156 @@ __device__ double block_max(double v)
     return v;
 }
 
-// GET_DT_BLOCK_ACM of active block k.  WAVES 1: one wavefront per block
-// (four blocks per workgroup; the 2D blocks' few hundred points), 0: the
-// whole workgroup per block.  The max and min are exact whatever the order,
-// so the per-group minimum may be combined in any grouping.
-template <int WAVES>
+// dt clamps of calculate_time_step.f90:58-118 on the device, so that a whole
+// step can be replayed from a hipGraph without a host round trip, and the
+// time advance of the step that takes this dt (its stages read DS_DT only).
+__device__ void dt_finalize(double *scal, double dtmin, const TimeDev &tc)
+{
+    const double time = scal[DS_TIME];
+    double dt;
+    if (tc.dt_fixed > 0.0) {
+        dt = tc.dt_fixed;
+    } else {
+        dt = dtmin;
+        if (tc.dt_max > 0.0) dt = fmin(tc.dt_max, dt);
+    }
+    if (tc.write_fixed_time) {
+        if (fmod(time + dt, tc.write_time) < fmod(time + 1e-12, tc.write_time) &&
+            !(fabs(fmod(time, tc.write_time)) < 1e-12) && time + 1e-12 > tc.write_time_first)
+            dt = tc.write_time - fmod(time, tc.write_time);
+    }
+    if (tc.write_backup_n > 0) {
+        const double wb = tc.write_backup_time;
+        if (fmod(time + dt, wb) < fmod(time + 1e-12, wb) && !(fabs(fmod(time, wb)) < 1e-12))
+            dt = wb - fmod(time, wb);
+    }
+    if (tc.use_stats) {
+        const double ts = tc.tsave_stats;
+        if (fmod(time + dt, ts) < fmod(time + 1e-12, ts) && !(fabs(fmod(time, ts)) < 1e-12))
+            dt = ts - fmod(time, ts);
+    }
+    if (time + dt > tc.time_max && time <= tc.time_max) dt = tc.time_max - time;
+    if (!(time < tc.time_max)) dt = 0.0;  // main.f90:293 loop condition
+    scal[DS_DT] = dt;
+    if (dt > 0.0) {
+        scal[DS_TIME] = time + dt;
+        scal[DS_ITER] = scal[DS_ITER] + 1.0;
+    }
+}
+
+// The minimum over all active blocks of a launch without groups: every
+// workgroup adds its minimum to DS_DTACC; the one that counts the last hands
+// the result on (DS_DTMIN_BITS; with STEP also dt_finalize) and leaves the
+// accumulator and the counter as it found them.  One launch instead of four
+// (clear, reduce, clamps, time advance): for small grids each of them cost as
+// much as a stage.
+template <bool STEP>
+__device__ void dt_combine(double *scal, double v, const TimeDev &tc)
+{
+    unsigned long long *acc = (unsigned long long *)(scal + DS_DTACC), *cnt = (unsigned long long *)(scal + DS_DTCNT);
+    if (v < DT_NONE)
+        __hip_atomic_fetch_min(acc, (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_fetch_add(cnt, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT) + 1 != gridDim.x) return;
+    const double m = __longlong_as_double(
+        (long long)__hip_atomic_exchange(acc, (unsigned long long)__double_as_longlong(DT_NONE), __ATOMIC_ACQ_REL,
+                                         __HIP_MEMORY_SCOPE_AGENT));
+    __hip_atomic_store(cnt, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    scal[DS_DTMIN_BITS] = m;
+    if constexpr (STEP) dt_finalize(scal, m, tc);
+}
+
+// GET_DT_BLOCK_ACM of the active blocks.  WAVES 1: a wavefront per block, four
+// blocks per workgroup at a time (2D blocks of a few hundred points), 0: the
+// workgroup per block; a workgroup goes on to the next ones until all are
+// done.  Four points per lane are requested at a time.  The max and min are
+// exact whatever the order, so the minimum may be combined in any grouping:
+// per group with grp (into dtmin[group]), else over the launch (dt_combine).
+template <int WAVES, bool STEP>
 __global__ __launch_bounds__(256) void k_dt(const double *__restrict__ in,
                                             const int32_t *__restrict__ act,
                                             const double *__restrict__ x0dx, Geo G, AcmDev a0,
                                             unsigned long long *dtmin, const int32_t *__restrict__ grp,
-                                            const AcmDev *__restrict__ gacm, int nact)
+                                            const AcmDev *__restrict__ gacm, int nact, double *scal, TimeDev tc)
 {
     const int lane = WAVES ? (int)(threadIdx.x & 63) : (int)threadIdx.x, step = WAVES ? 64 : (int)blockDim.x;
     const int w = (int)(threadIdx.x >> 6);
-    const int k = WAVES ? (int)blockIdx.x * 4 + w : (int)blockIdx.x;
-    const bool live = !WAVES || k < nact;  // wave-uniform
-    double dt = 0.0;
-    if (live) {
-        const int b = act[k];
-        const int npts = G.bs0 * G.bs1 * G.bs2;
-        const int zoff = (G.bs2 > 1) ? G.g : 0;
-        const double *u = in + (size_t)b * G.blk;
-        double m = -1.0;
-        for (int p = lane; p < npts; p += step) {
-            const int ix = p % G.bs0, iy = (p / G.bs0) % G.bs1, iz = p / (G.bs0 * G.bs1);
-            const size_t i = ((size_t)(zoff + iz) * G.ny + (G.g + iy)) * G.nx + (G.g + ix);
-            double v = u[i] * u[i] + u[G.cs + i] * u[G.cs + i];
-            if (G.bs2 > 1) v = v + u[2 * G.cs + i] * u[2 * G.cs + i];
-            m = fmax(m, v);
-        }
-        m = WAVES ? wave_max(m) : block_max(m);
-        if (lane == 0) {
-            const AcmDev &a = gacm ? gacm[grp[k]] : a0;  // per-group constants of independent forests
-            double dxmin = x0dx[6 * k + 3];
-            for (int d = 1; d < a.dim; ++d) dxmin = fmin(dxmin, x0dx[6 * k + 3 + d]);
-            const double ueig = sqrt(m) + sqrt(a.c_0 * a.c_0 + m);
-            dt = (ueig >= 1.0e-6) ? a.CFL * dxmin / ueig : 1.0e-2;
-            if (a.nu > 1.0e-13) dt = fmin(dt, a.CFL_nu * (dxmin * dxmin) / a.nu);
-            if (a.gamma_p > 0.0) dt = fmin(dt, a.CFL_eta * a.gamma_p);
-            if (a.penal) dt = fmin(dt, a.CFL_eta * a.C_eta);
-            if (a.sponge) dt = fmin(dt, a.CFL_eta * a.C_sponge);
-            if (!WAVES) atomicMin(grp ? dtmin + grp[k] : dtmin, (unsigned long long)__double_as_longlong(dt));
-        }
-    }
-    if (WAVES) {
-        // the workgroup's four blocks (consecutive active entries: mostly one
-        // group) combined first, one atomic per distinct group
-        __shared__ double sdt[4];
-        __shared__ int sgr[4];
-        if (lane == 0) {
-            sdt[w] = dt;
-            sgr[w] = live ? (grp ? grp[k] : 0) : -1;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0)
-            for (int x = 0; x < 4; ++x) {
-                if (sgr[x] < 0) continue;
-                bool first = true;
-                for (int y = 0; y < x; ++y) first = first && sgr[y] != sgr[x];
-                if (!first) continue;
-                double v = sdt[x];
-                for (int y = x + 1; y < 4; ++y)
-                    if (sgr[y] == sgr[x]) v = fmin(v, sdt[y]);
-                atomicMin(dtmin + sgr[x], (unsigned long long)__double_as_longlong(v));
+    const int nxy = G.bs0 * G.bs1, npts = nxy * G.bs2, zoff = (G.bs2 > 1) ? G.g : 0;
+    double all = DT_NONE;  // the minimum of this wavefront's (workgroup's) blocks, in lane 0
+    for (int k0 = (int)blockIdx.x * (WAVES ? 4 : 1); k0 < nact; k0 += (int)gridDim.x * (WAVES ? 4 : 1)) {
+        const int k = k0 + (WAVES ? w : 0);
+        const bool live = k < nact;  // wave-uniform
+        double dt = DT_NONE;
+        if (live) {
+            const double *u = in + (size_t)act[k] * G.blk;
+            double m = -1.0;
+            for (int p0 = lane; p0 < npts; p0 += 4 * step) {
+                double v[4][3];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int p = min(p0 + j * step, npts - 1);  // the last point again past the end
+                    const int iz = G.bs2 > 1 ? p / nxy : 0, r = p - iz * nxy, iy = r / G.bs0, ix = r - iy * G.bs0;
+                    const size_t i = ((size_t)(zoff + iz) * G.ny + (G.g + iy)) * G.nx + (G.g + ix);
+                    v[j][0] = u[i];
+                    v[j][1] = u[G.cs + i];
+                    v[j][2] = G.bs2 > 1 ? u[2 * G.cs + i] : 0.0;
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    double s = v[j][0] * v[j][0] + v[j][1] * v[j][1];
+                    if (G.bs2 > 1) s = s + v[j][2] * v[j][2];
+                    m = fmax(m, s);
+                }
             }
+            m = WAVES ? wave_max(m) : block_max(m);
+            if (lane == 0) {
+                const AcmDev &a = gacm ? gacm[grp[k]] : a0;  // per-group constants of independent forests
+                double dxmin = x0dx[6 * k + 3];
+                for (int d = 1; d < a.dim; ++d) dxmin = fmin(dxmin, x0dx[6 * k + 3 + d]);
+                const double ueig = sqrt(m) + sqrt(a.c_0 * a.c_0 + m);
+                dt = (ueig >= 1.0e-6) ? a.CFL * dxmin / ueig : 1.0e-2;
+                if (a.nu > 1.0e-13) dt = fmin(dt, a.CFL_nu * (dxmin * dxmin) / a.nu);
+                if (a.gamma_p > 0.0) dt = fmin(dt, a.CFL_eta * a.gamma_p);
+                if (a.penal) dt = fmin(dt, a.CFL_eta * a.C_eta);
+                if (a.sponge) dt = fmin(dt, a.CFL_eta * a.C_sponge);
+                if (!WAVES && grp) atomicMin(dtmin + grp[k], (unsigned long long)__double_as_longlong(dt));
+                all = fmin(all, dt);
+            }
+        }
+        if (!WAVES) {
+            __syncthreads();  // block_max's shared memory is reused
+        } else if (grp) {
+            // the workgroup's four blocks (consecutive active entries: mostly one
+            // group) combined first, one atomic per distinct group
+            __shared__ double sdt[4];
+            __shared__ int sgr[4];
+            __syncthreads();
+            if (lane == 0) {
+                sdt[w] = dt;
+                sgr[w] = live ? grp[k] : -1;
+            }
+            __syncthreads();
+            if (threadIdx.x == 0)
+                for (int x = 0; x < 4; ++x) {
+                    if (sgr[x] < 0) continue;
+                    bool first = true;
+                    for (int y = 0; y < x; ++y) first = first && sgr[y] != sgr[x];
+                    if (!first) continue;
+                    double v = sdt[x];
+                    for (int y = x + 1; y < 4; ++y)
+                        if (sgr[y] == sgr[x]) v = fmin(v, sdt[y]);
+                    atomicMin(dtmin + sgr[x], (unsigned long long)__double_as_longlong(v));
+                }
+        }
     }
+    if (grp) return;
+    if (WAVES) {
+        __shared__ double part[4];
+        if (lane == 0) part[w] = all;
+        __syncthreads();
+        all = fmin(fmin(part[0], part[1]), fmin(part[2], part[3]));
+    }
+    if (threadIdx.x == 0) dt_combine<STEP>(scal, all, tc);
 }
 
 __global__ __launch_bounds__(256) void k_maxabs(const double *__restrict__ in,
@@ -1776,21 +1861,29 @@ __global__ void k_scalar_init(double *scal, int which, double v)
     if (threadIdx.x == 0) scal[which] = v;
 }
 
-int launch_dt(wh_pool *P, const AcmDev &a)
+// Blocks of up to 600 points: a wavefront each (with the read-back, 4096
+// blocks of 24^2: 38 us, by workgroups 50; 64 of 32^2: 21.7, by workgroups
+// 20.4).
+static bool dt_by_waves(const Geo &G) { return G.bs0 * G.bs1 * G.bs2 <= 600; }
+
+int launch_dt(wh_pool *P, const AcmDev &a, const TimeDev *step)
 {
-    hipLaunchKernelGGL(k_scalar_init, dim3(1), dim3(64), 0, P->stream, P->scal, (int)DS_DTMIN_BITS,
-                       9.0e9);
-    if (P->nact > 0) {
-        const Geo G = make_geo(P);
-        if (P->d.dim == 2)
-            hipLaunchKernelGGL(k_dt<1>, dim3((P->nact + 3) / 4), dim3(256), 0, P->stream, P->block, P->d_active,
-                               P->d_x0dx, G, a, (unsigned long long *)(P->scal + DS_DTMIN_BITS),
-                               (const int32_t *)nullptr, (const AcmDev *)nullptr, P->nact);
-        else
-            hipLaunchKernelGGL(k_dt<0>, dim3(P->nact), dim3(256), 0, P->stream, P->block, P->d_active,
-                               P->d_x0dx, G, a, (unsigned long long *)(P->scal + DS_DTMIN_BITS),
-                               (const int32_t *)nullptr, (const AcmDev *)nullptr, P->nact);
-    }
+    const Geo G = make_geo(P);
+    const TimeDev tc = step ? *step : TimeDev{};
+    const bool waves = dt_by_waves(G);
+    // At most 1 (wavefronts) or 2 (workgroups per block) workgroups per compute
+    // unit, as each ends with a release of its own: 4096 blocks of 16^2 31 / 33
+    // / 44 us with 1 / 2 / 4, of 24^3 344 / 314 / 335 us.
+    const dim3 grid(std::max(1, waves ? std::min(P->n_cu, (P->nact + 3) / 4) : std::min(2 * P->n_cu, P->nact)));
+#define LDT(W, ST)                                                                                                 \
+    hipLaunchKernelGGL((k_dt<W, ST>), grid, dim3(256), 0, P->stream, P->block, P->d_active, P->d_x0dx, G, a,        \
+                       (unsigned long long *)nullptr, (const int32_t *)nullptr, (const AcmDev *)nullptr, P->nact, \
+                       P->scal, tc)
+    if (waves && step) LDT(1, true);
+    else if (waves) LDT(1, false);
+    else if (step) LDT(0, true);
+    else LDT(0, false);
+#undef LDT
     WH_HIP(hipGetLastError());
     return WH_OK;
 }
@@ -1804,20 +1897,21 @@ __global__ void k_fill_u64(unsigned long long *p, int n, unsigned long long v)
 int launch_dt_groups(wh_pool *P, const AcmDev &a)
 {
     const int n = P->ngrp;
-    const double init = 9.0e9;
     unsigned long long bits;
-    std::memcpy(&bits, &init, sizeof bits);
+    std::memcpy(&bits, &DT_NONE, sizeof bits);
     hipLaunchKernelGGL(k_fill_u64, dim3((n + 255) / 256), dim3(256), 0, P->stream, P->d_dtg, n,
                        bits);
     if (P->nact > 0) {
         const Geo G = make_geo(P);
         const AcmDev *gacm = P->ngacm == P->ngrp ? P->d_gacm : nullptr;
-        if (P->d.dim == 2)
-            hipLaunchKernelGGL(k_dt<1>, dim3((P->nact + 3) / 4), dim3(256), 0, P->stream, P->block, P->d_active,
-                               P->d_x0dx, G, a, P->d_dtg, (const int32_t *)P->d_grp, gacm, P->nact);
+        const bool waves = dt_by_waves(G);
+        const dim3 grid(waves ? (P->nact + 3) / 4 : P->nact);
+        if (waves)
+            hipLaunchKernelGGL((k_dt<1, false>), grid, dim3(256), 0, P->stream, P->block, P->d_active, P->d_x0dx, G, a,
+                               P->d_dtg, (const int32_t *)P->d_grp, gacm, P->nact, P->scal, TimeDev{});
         else
-            hipLaunchKernelGGL(k_dt<0>, dim3(P->nact), dim3(256), 0, P->stream, P->block, P->d_active,
-                               P->d_x0dx, G, a, P->d_dtg, (const int32_t *)P->d_grp, gacm, P->nact);
+            hipLaunchKernelGGL((k_dt<0, false>), grid, dim3(256), 0, P->stream, P->block, P->d_active, P->d_x0dx, G, a,
+                               P->d_dtg, (const int32_t *)P->d_grp, gacm, P->nact, P->scal, TimeDev{});
     }
     WH_HIP(hipGetLastError());
     return WH_OK;
@@ -1836,57 +1930,18 @@ int launch_maxabs(wh_pool *P, const double *in)
     return WH_OK;
 }
 
-// dt clamps of calculate_time_step.f90:58-118 on the device, so that a whole
-// step can be replayed from a hipGraph without a host round trip.
-__global__ void k_dt_finalize(double *scal, TimeDev tc)
+// time, iteration and dt of the device-side time loop in one launch
+__global__ void k_time_set(double *scal, double time, double iter)
 {
     if (threadIdx.x != 0) return;
-    const double time = scal[DS_TIME];
-    double dt;
-    if (tc.dt_fixed > 0.0) {
-        dt = tc.dt_fixed;
-    } else {
-        dt = scal[DS_DTMIN_BITS];  // the min was taken on the bit pattern of positive doubles
-        if (tc.dt_max > 0.0) dt = fmin(tc.dt_max, dt);
-    }
-    if (tc.write_fixed_time) {
-        if (fmod(time + dt, tc.write_time) < fmod(time + 1e-12, tc.write_time) &&
-            !(fabs(fmod(time, tc.write_time)) < 1e-12) && time + 1e-12 > tc.write_time_first)
-            dt = tc.write_time - fmod(time, tc.write_time);
-    }
-    if (tc.write_backup_n > 0) {
-        const double wb = tc.write_backup_time;
-        if (fmod(time + dt, wb) < fmod(time + 1e-12, wb) && !(fabs(fmod(time, wb)) < 1e-12))
-            dt = wb - fmod(time, wb);
-    }
-    if (tc.use_stats) {
-        const double ts = tc.tsave_stats;
-        if (fmod(time + dt, ts) < fmod(time + 1e-12, ts) && !(fabs(fmod(time, ts)) < 1e-12))
-            dt = ts - fmod(time, ts);
-    }
-    if (time + dt > tc.time_max && time <= tc.time_max) dt = tc.time_max - time;
-    if (!(time < tc.time_max)) dt = 0.0;  // main.f90:293 loop condition
-    scal[DS_DT] = dt;
+    scal[DS_TIME] = time;
+    scal[DS_ITER] = iter;
+    scal[DS_DT] = 0.0;
 }
 
-__global__ void k_time_advance(double *scal)
+int launch_time_set(wh_pool *P, double time, double iter)
 {
-    if (threadIdx.x == 0 && scal[DS_DT] > 0.0) {
-        scal[DS_TIME] = scal[DS_TIME] + scal[DS_DT];
-        scal[DS_ITER] = scal[DS_ITER] + 1.0;
-    }
-}
-
-int launch_dt_finalize(wh_pool *P, const TimeDev &tc)
-{
-    hipLaunchKernelGGL(k_dt_finalize, dim3(1), dim3(64), 0, P->stream, P->scal, tc);
-    WH_HIP(hipGetLastError());
-    return WH_OK;
-}
-
-int launch_time_advance(wh_pool *P)
-{
-    hipLaunchKernelGGL(k_time_advance, dim3(1), dim3(64), 0, P->stream, P->scal);
+    hipLaunchKernelGGL(k_time_set, dim3(1), dim3(64), 0, P->stream, P->scal, time, iter);
     WH_HIP(hipGetLastError());
     return WH_OK;
 }
