@@ -699,12 +699,10 @@ __global__ __launch_bounds__(256) void k_xyplane(const double *in, double *out, 
 // plane is requested before the current one is worked on, and what a plane
 // yields is stored just before that request, so that waiting for the loads
 // (which waits for the stores before them too) finds both done.
-// copy, init_copy: as in k_xyplane.
 constexpr int XYZ_PRE = 4;  // plane values per thread (the host checks that they suffice)
 template <int OP, int X, int Y>
-__global__ __launch_bounds__(1024) void k_xyz(const double *in, double *out, double *copy,
-                                              const int32_t *__restrict__ ids, XfGeo G, int bs2, int init_copy,
-                                              FixedCoef C)
+__global__ __launch_bounds__(1024) void k_xyz(const double *__restrict__ in, double *__restrict__ out,
+                                              const int32_t *__restrict__ ids, XfGeo G, int bs2, FixedCoef C)
 {
     constexpr FixedChain K = fixed_chain<OP, X, Y>();
     constexpr int WN = K.hi - K.lo + 1;
@@ -715,23 +713,7 @@ __global__ __launch_bounds__(1024) void k_xyz(const double *in, double *out, dou
     const size_t b = (size_t)ids[k];
     const double *src = in + b * G.blk_in + (size_t)c * G.cs;
     double *dst = out + b * G.blk_out + (size_t)c * G.cs;
-    double *cpy = copy ? copy + b * G.blk_copy + (size_t)c * G.cs : nullptr;
     const int rows = G.bs1 + 2 * G.ext;
-    int outside = 0;  // bit j: this thread's j-th plane value lies where no pass writes
-    if (init_copy)
-        for (int j = 0; j < XYZ_PRE; ++j) {
-            const int i = tid + j * nt, y = i / G.nx, x = i - y * G.nx - G.g, r = y - (G.g - G.ext);
-            if (i < nxy && (x < 0 || x >= G.bs0 || r < 0 || r >= rows)) outside |= 1 << j;
-        }
-    if (cpy || init_copy)
-        for (int z = 0; z < G.nz; ++z) {  // the planes outside the passes
-            if (z >= G.z0 && z < G.z1) continue;
-            for (int i = tid; i < nxy; i += nt) {
-                const double v = src[z * nxy + i];
-                if (cpy) cpy[z * nxy + i] = v;
-                if (init_copy) dst[z * nxy + i] = v;
-            }
-        }
     // this thread's (x, y) point: even rows first, then odd rows
     const int yA = (G.bs1 + 1) / 2, pa = (yA * G.bs0 + 63) & ~63;
     const bool odd = __builtin_amdgcn_readfirstlane(tid >= pa ? 1 : 0);
@@ -764,11 +746,7 @@ __global__ __launch_bounds__(1024) void k_xyz(const double *in, double *out, dou
 #pragma unroll
         for (int j = 0; j < XYZ_PRE; ++j) {
             const int i = tid + j * nt;
-            if (i < nxy) {
-                S[i] = pre[j];
-                if (cpy) cpy[z * nxy + i] = pre[j];
-                if (outside >> j & 1) dst[z * nxy + i] = pre[j];
-            }
+            if (i < nxy) S[i] = pre[j];
         }
         if (z > G.z0) store(z - 1);
         load(min(z + 1, G.z1 - 1));
@@ -1312,12 +1290,12 @@ int launch_xform_xy(wh_pool *P, const double *in, size_t blk_in, double *out, si
     // kernel, CDF44: 512 blocks of 24^3 548 / 679 us, of 20^3 391 / 476,
     // 1024 of 16^3 505 / 618, 256 of 24^3 309 / 324, but 64 of 24^3 78 / 59;
     // CDF22, 256 of 24^3: 179 / 134; CDF40 reconstruction (whole rows), 512 of
-    // 24^3: 479 / 346.
+    // 24^3: 479 / 346; in place with the copy, CDF44, 512 of 24^3: 818 / 684.
     const int items = (((bs1 + 1) / 2 * bs0 + 63) & ~63) + bs1 / 2 * bs0, nt = (items + 63) & ~63;
-    if (dim == 3 && X >= 4 && !init_copy && nt <= 1024 && nxy <= XYZ_PRE * nt &&
+    if (dim == 3 && X >= 4 && !init_copy && !copy && nt <= 1024 && nxy <= XYZ_PRE * nt &&
         (long)nb * P->d.neq >= 4L * P->n_cu) {
-        hipLaunchKernelGGL((k_xyz<OP, X, Y>), dim3((unsigned)(nb * P->d.neq)), dim3(nt), lds, P->stream, in, out, copy,
-                           P->ws.cur_ids, G, bs2, init_copy ? 1 : 0, C);
+        hipLaunchKernelGGL((k_xyz<OP, X, Y>), dim3((unsigned)(nb * P->d.neq)), dim3(nt), lds, P->stream, in, out,
+                           P->ws.cur_ids, G, bs2, C);
         WH_HIP(hipGetLastError());
         return WH_OK;
     }
