@@ -153,7 +153,7 @@ static int build_faces(wh_pool *P, int R)
     FaceGather &F = P->faces;
     const PatchSet &ps = P->ps[0];
     const int dim = P->d.dim, nf = 2 * dim, g = P->d.g;
-    F.any = false;
+    F.any = F.whole = false;
     F.h_kept.clear();
     F.h_chunks.clear();
     F.h_face.assign((size_t)P->nact * nf, -1);
@@ -221,6 +221,7 @@ static int build_faces(wh_pool *P, int R)
             F.h_kept.push_back(q);
         }
     }
+    F.whole = F.h_kept.empty() && std::find(F.h_face.begin(), F.h_face.end(), -1) == F.h_face.end();
     F.stage_begin[4] = (int)F.h_kept.size();
     F.chunk_begin[4] = (int)F.h_chunks.size();
     if (F.h_face.size() > F.cap_face || F.h_kept.size() > F.cap_kept || F.h_chunks.size() > F.cap_chunks)
@@ -303,8 +304,7 @@ static int sync_kept(wh_pool *P, const FaceGather &F, double *arr)
 // one step of the fused path; dt is taken from the device scalar DS_DT, or
 // per block from dtb (block groups).  With a 2D face table no ghost fill is
 // launched: every stage reads its blocks' halos from the neighbours'
-// interiors of its input array.  With a 3D face table the state
-// gets its ghost fill as without it (its ghost nodes are the caller's); of
+// interiors of its input array.  With a 3D face table the state gets its ghost fill as without it (its ghost nodes are the caller's); of
 // the fills of the stage inputs in the work slots only the kept patches run.
 static int fused_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
                       const double *dtb = nullptr)
@@ -316,6 +316,9 @@ static int fused_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
                     array_ptr(P, WH_WORK + 2, nullptr, nullptr)};
     const FaceGather *fg = face_table(P, a);
     const bool of_state = P->d.dim == 2;  // whether the first stage, too, uses the face table
+    // 3D with every face gathered: the stage inputs need no ghost nodes and
+    // are held without them, in rows that fill cache lines
+    const bool compact = fg && !of_state && fg->whole;
     // the ghost fill (timed as a sync launch)
     auto sync = [&](double *arr) {
         const bool faces = fg && (of_state || arr != S);
@@ -325,7 +328,8 @@ static int fused_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
     auto launch_fused_stage = [&](wh_pool *Q, const AcmDev &aa, const double *tin, double *tout, const double *u0,
                                   double *ac, double *sout, int mode, double acoef, double bcoef, const double *db) {
         return wh::launch_fused_stage(Q, aa, tin, tout, u0, ac, sout, mode, acoef, bcoef, db,
-                                      fg && (of_state || tin != S) ? fg->d_face : nullptr);
+                                      fg && (of_state || tin != S) ? fg->d_face : nullptr, compact && tin != S,
+                                      compact);
     };
     int rc;
     if ((rc = sync(S))) return rc;
@@ -1224,6 +1228,7 @@ int wh_time_stage_kernel(wh_pool *P, const wh_acm_params *p, int reps, double *m
     // the launches gather their halos the same way
     if (int rc = update_faces(P, a)) return rc;
     const FaceGather *fg = face_table(P, a);
+    const bool compact = fg && P->d.dim == 3 && fg->whole;
     auto rk4 = [&]() -> int {
         const double ca[4] = {0.5, 0.5, 1.0, 0.0}, cb[4] = {1.0 / 6.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0};
         const int mode[4] = {0, 1, 1, 2};
@@ -1231,7 +1236,8 @@ int wh_time_stage_kernel(wh_pool *P, const wh_acm_params *p, int reps, double *m
             if (int rc = launch_fused_stage(P, a, P->block, mode[j] == 2 ? nullptr : tout,
                                             mode[j] == 1 ? P->block : nullptr, acc, mode[j] == 2 ? sout : nullptr,
                                             mode[j], ca[j], cb[j], nullptr,
-                                            fg && (P->d.dim == 2 || j > 0) ? fg->d_face : nullptr))
+                                            fg && (P->d.dim == 2 || j > 0) ? fg->d_face : nullptr,
+                                            compact && j > 0, compact))
                 return rc;
         return WH_OK;
     };
@@ -1284,14 +1290,17 @@ int wh_autotune(wh_pool *P, const wh_acm_params *p, int reps, int *best_value, d
     double *acc = array_ptr(P, WH_WORK + 0, nullptr, nullptr);
     auto launch = [&]() -> int {
         const int32_t *faces = nullptr;
+        bool compact = false;
         if (fused && three) {
             if (int rc = update_faces(P, a)) return rc;
             const FaceGather *fg = face_table(P, a);
             if (int rc = fg ? sync_kept(P, *fg, out) : launch_sync(P, 0, out, -1)) return rc;
             faces = fg ? fg->d_face : nullptr;
+            compact = fg && fg->whole;
         }
         if (fused)
-            return launch_fused_stage(P, a, P->block, out, P->block, acc, nullptr, 1, 0.5, 1.0 / 3.0, nullptr, faces);
+            return launch_fused_stage(P, a, P->block, out, P->block, acc, nullptr, 1, 0.5, 1.0 / 3.0, nullptr, faces,
+                                      compact, compact);
         return launch_rhs(P, a, P->block, out, P->d_active, P->d_x0dx, P->nact);
     };
     const Var saved{knob, P->k3d_zsplit, P->k3d_waves, P->k3d_xcd};

@@ -185,6 +185,7 @@ struct FaceGather {
     uint64_t topo = ~0ull;  // topology version and stencil reach it was built for
     int reach = 0;
     bool any = false;       // at least one face is gathered
+    bool whole = false;     // every face is gathered and no patch is kept
     std::vector<int32_t> h_face;  // 2*dim ids per active position: -x, +x, -y, +y (, -z, +z); -1: own ghost nodes
     int32_t *d_face = nullptr;
     size_t cap_face = 0;
@@ -276,10 +277,13 @@ int launch_combine(wh_pool *P, double *out, const double *base, int nterms,
 int launch_dt(wh_pool *P, const AcmDev &a, const TimeDev *step = nullptr);
 int launch_maxabs(wh_pool *P, const double *in);
 // dtb: per active-list position dt (block groups), or null for the pool's DS_DT
-// gnb: the face table (FaceGather; 3D: of the z-marching kernel), or null
+// gnb: the face table (FaceGather; 3D: of the z-marching kernel), or null;
+// in_compact, out_compact: tin / tout hold block interiors only, as the
+// accumulator does (3D, where every face is gathered)
 int launch_fused_stage(wh_pool *P, const AcmDev &a, const double *tin, double *tout,
                        const double *u0, double *acc, double *sout, int mode, double acoef,
-                       double bcoef, const double *dtb, const int32_t *gnb = nullptr);
+                       double bcoef, const double *dtb, const int32_t *gnb = nullptr, bool in_compact = false,
+                       bool out_compact = false);
 // per-group minimum block dt into P->d_dtg (bit patterns) for the P->ngrp groups
 int launch_dt_groups(wh_pool *P, const AcmDev &a);
 // whether the 3D stages run the z-marching kernel (the one that can gather)

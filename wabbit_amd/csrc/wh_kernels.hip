@@ -208,6 +208,9 @@ struct StageArgs {
     // halo gather: the senders of each block's 4 (2D) or 6 faces by active
     // position (-1: own ghost nodes), or null
     const int32_t *gnb;
+    // 3D z-marching kernel: the stage input / the next stage input hold block
+    // interiors only, laid out as the accumulator
+    int in_compact, out_compact;
 };
 
 struct NoEpilogue {};
@@ -224,7 +227,8 @@ template <int NC>
 __device__ __forceinline__ StageBlk stage_blk(const StageArgs &sa, int b, size_t blk, int npts)
 {
     const size_t o = (size_t)b * blk;
-    return StageBlk{sa.u0 ? sa.u0 + o : nullptr, sa.acc + (size_t)b * NC * npts, sa.tout ? sa.tout + o : nullptr,
+    const size_t oc = (size_t)b * NC * npts;
+    return StageBlk{sa.u0 ? sa.u0 + o : nullptr, sa.acc + oc, sa.tout ? sa.tout + (sa.out_compact ? oc : o) : nullptr,
                     sa.sout ? sa.sout + o : nullptr};
 }
 
@@ -253,12 +257,14 @@ __device__ __forceinline__ void stage_epilogue(const StageArgs &sa, const StageB
 }
 
 // the fused epilogue with the acc / u0 values of the point already loaded
-// (accv, u0v: one value per component)
-template <int NC>
+// (accv, u0v: one value per component); with COMPACT the next stage input may
+// be laid out as the accumulator
+template <int NC, bool COMPACT = false>
 __device__ __forceinline__ void stage_epilogue_pre(const StageArgs &sa, const StageBlk &B, int k, int gi, int cs,
                                                    int p, int npts, const double *r, const double *ucen,
                                                    ptrdiff_t ucs, const double *accv, const double *u0v)
 {
+    const int ti = COMPACT && sa.out_compact ? p : gi, tcs = COMPACT && sa.out_compact ? npts : cs;
     const double dt = sa.dtb ? sa.dtb[k] : sa.scal[DS_DT];
     const double ca = dt * sa.a, cb = dt * sa.b;
 #pragma unroll
@@ -267,10 +273,10 @@ __device__ __forceinline__ void stage_epilogue_pre(const StageArgs &sa, const St
         if (sa.mode == 0) {
             const double u0 = ucen[c * ucs];
             B.acc[ia] = sa.use_b ? u0 + cb * r[c] : u0;
-            if (sa.use_a) B.tout[i] = u0 + ca * r[c];
+            if (sa.use_a) B.tout[ti + c * tcs] = u0 + ca * r[c];
         } else if (sa.mode == 1) {
             if (sa.use_b) B.acc[ia] = accv[c] + cb * r[c];
-            if (sa.use_a) B.tout[i] = u0v[c] + ca * r[c];
+            if (sa.use_a) B.tout[ti + c * tcs] = u0v[c] + ca * r[c];
         } else {
             B.sout[i] = sa.use_b ? accv[c] + cb * r[c] : accv[c];
         }
@@ -660,10 +666,11 @@ __global__ __launch_bounds__(256) void k_rhs3d_multi(const MPoolDev *__restrict_
 // +y, -z, +z), or from the block's own ghost nodes where the id is -1;
 // without it always from the ghost nodes.  The stencils run along the axes,
 // so edges and corners are not read.
-// Bound by the memory system: over 4096 24^3 blocks (FD4, g 6, middle and
-// outer stages of RK4) 2.26 ms a launch for 9.2 GB = 4.1 TB/s, where a large
-// copy reaches 4.4 (before: 4.34 ms, and 3.30 ms by the flat kernel); over
-// 512 blocks 0.29 ms (0.56, 0.42).
+// Bound by the memory system: over 4096 24^3 blocks (FD4, g 6, the stages of
+// RK4) 2.26 ms a launch for 9.2 GB = 4.1 TB/s (before: 4.34 ms, and 3.30 ms by
+// the flat kernel); with the stage inputs held without ghost nodes, in rows
+// that fill cache lines, 1.92 ms = 4.8 TB/s, where a large copy reaches 4.4.
+// Over 512 blocks 0.29 and 0.25 ms (0.56, 0.42).
 template <int S, bool SKEW, bool FUSED>
 __global__ __launch_bounds__(512) void k_rhs3d_zm(const double *__restrict__ in,
                                                   double *__restrict__ out,
@@ -687,19 +694,23 @@ __global__ __launch_bounds__(512) void k_rhs3d_zm(const double *__restrict__ in,
     const int tid = threadIdx.x;
     const int iyl = tid / G.bs0, ix = tid - iyl * G.bs0, iy = y0 + iyl;
     const int tx = G.bs0 + 2 * R, ty = ty0 + 2 * R, tcs = tx * ty;
-    const int zs = G.nx * G.ny, cs = (int)G.cs;
-    const double *u = in + (size_t)b * G.blk;
+    const int zs = G.nx * G.ny, cs = (int)G.cs, npts = G.bs0 * G.bs1 * G.bs2;
+    // the input's layout: ghost-including blocks, or interiors only
+    const bool ci = FUSED && sa.in_compact;
+    const int ig = ci ? 0 : G.g, inx = ci ? G.bs0 : G.nx, izs = ci ? G.bs0 * G.bs1 : zs, ics = ci ? npts : cs;
+    const size_t iblk = ci ? (size_t)4 * npts : G.blk;
+    const double *u = in + (size_t)b * iblk;
     // where the values beyond each face are read, relative to their place in
     // this block's ghost nodes
     ptrdiff_t fo[6] = {0, 0, 0, 0, 0, 0};
     if (FUSED && sa.gnb) {
         const int32_t *nb = sa.gnb + (size_t)k * 6;
-        const ptrdiff_t sh[3] = {G.bs0, (ptrdiff_t)G.bs1 * G.nx, (ptrdiff_t)G.bs2 * zs};
+        const ptrdiff_t sh[3] = {G.bs0, (ptrdiff_t)G.bs1 * inx, (ptrdiff_t)G.bs2 * izs};
 #pragma unroll
         for (int f = 0; f < 6; ++f)
-            if (nb[f] >= 0) fo[f] = ((ptrdiff_t)nb[f] - b) * (ptrdiff_t)G.blk + (f & 1 ? -sh[f >> 1] : sh[f >> 1]);
+            if (nb[f] >= 0) fo[f] = ((ptrdiff_t)nb[f] - b) * (ptrdiff_t)iblk + (f & 1 ? -sh[f >> 1] : sh[f >> 1]);
     }
-    const int col = (G.g + iy) * G.nx + (G.g + ix);
+    const int col = (G.g + iy) * G.nx + (G.g + ix), icol = (ig + iy) * inx + (ig + ix);
     const double dx0 = x0dx[6 * k + 3], dx1 = x0dx[6 * k + 4], dx2 = x0dx[6 * k + 5];
     const double inv[3] = {wave_uniform(1.0 / dx0), wave_uniform(1.0 / dx1), wave_uniform(1.0 / dx2)};
     const double inv2[3] = {wave_uniform(1.0 / (dx0 * dx0)), wave_uniform(1.0 / (dx1 * dx1)),
@@ -726,14 +737,13 @@ __global__ __launch_bounds__(512) void k_rhs3d_zm(const double *__restrict__ in,
             o = kk < R ? fo[0] : fo[1];
         }
         r_lds = py * tx + px;
-        r_src = u + o + (ptrdiff_t)(G.g + y0 - R + py) * G.nx + (G.g - R + px);
+        r_src = u + o + (ptrdiff_t)(ig + y0 - R + py) * inx + (ig - R + px);
     }
     // the slab's own points of plane iz (-R .. Bs2 + R - 1), component c
     auto own = [&](int iz, int c) -> double {
         const double *p = u + (iz < 0 ? fo[4] : iz >= G.bs2 ? fo[5] : (ptrdiff_t)0);
-        return p[c * cs + (G.g + iz) * zs + col];
+        return p[c * ics + (ig + iz) * izs + icol];
     };
-    const int npts = G.bs0 * G.bs1 * G.bs2;
     const StageBlk SB = FUSED ? stage_blk<4>(sa, b, G.blk, npts) : StageBlk{};
     double apre[4] = {0, 0, 0, 0}, upre[4] = {0, 0, 0, 0};
     double q[4][W];
@@ -746,7 +756,7 @@ __global__ __launch_bounds__(512) void k_rhs3d_zm(const double *__restrict__ in,
     for (int c = 0; c < 4; ++c) nq[c] = own(z0 + R, c);
     if (ringer)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) nr[c] = r_src[c * cs + (G.g + z0) * zs];
+        for (int c = 0; c < 4; ++c) nr[c] = r_src[c * ics + (ig + z0) * izs];
 
     const int lc = (iyl + R) * tx + (ix + R);
     for (int iz = z0; iz < z1; ++iz) {
@@ -775,7 +785,7 @@ __global__ __launch_bounds__(512) void k_rhs3d_zm(const double *__restrict__ in,
             for (int c = 0; c < 4; ++c) nq[c] = own(iz + 1 + R, c);
             if (ringer)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) nr[c] = r_src[c * cs + (G.g + iz + 1) * zs];
+                for (int c = 0; c < 4; ++c) nr[c] = r_src[c * ics + (ig + iz + 1) * izs];
         }
         __syncthreads();
         // x/y from the LDS plane, z from the register queue
@@ -787,8 +797,8 @@ __global__ __launch_bounds__(512) void k_rhs3d_zm(const double *__restrict__ in,
         acm_point<3, S, SKEW>(A, inv, inv2, a, MaskMem{mk ? mk + gi : nullptr, (ptrdiff_t)G.cs}, r);
         if constexpr (FUSED) {
             const double u0c[4] = {q[0][R], q[1][R], q[2][R], q[3][R]};
-            stage_epilogue_pre<4>(sa, SB, k, gi, cs, pnt, npts, r, u0c, 1, apre, upre);
-            stage_ghost_cols<4>(sa, SB, gi - (G.g + ix), cs, ix, G.bs0, G.g);
+            stage_epilogue_pre<4, true>(sa, SB, k, gi, cs, pnt, npts, r, u0c, 1, apre, upre);
+            if (!sa.out_compact) stage_ghost_cols<4>(sa, SB, gi - (G.g + ix), cs, ix, G.bs0, G.g);
         } else {
             double *o = out + (size_t)b * G.blk + gi;
 #pragma unroll
@@ -994,10 +1004,12 @@ int launch_rhs(wh_pool *P, const AcmDev &a, const double *in, double *out, const
 
 int launch_fused_stage(wh_pool *P, const AcmDev &a, const double *tin, double *tout,
                        const double *u0, double *acc, double *sout, int mode, double acoef,
-                       double bcoef, const double *dtb, const int32_t *gnb)
+                       double bcoef, const double *dtb, const int32_t *gnb, bool in_compact, bool out_compact)
 {
     StageArgs sa{};
     sa.gnb = gnb;
+    sa.in_compact = in_compact;
+    sa.out_compact = out_compact;
     sa.dtb = dtb;
     sa.u0 = u0;
     sa.acc = acc;
