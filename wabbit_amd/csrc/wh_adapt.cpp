@@ -157,6 +157,7 @@ struct Tree {
             wq[d] = q[d] & (m - 1);  // periodic wrap; m is a power of two
         }
         if (level < (int)dense.size() && !dense[level].empty()) return dense[level][lin(level, wq)];
+        if (map.empty()) return -1;
         auto it = map.find(qkey(level, wq));
         return it == map.end() ? -1 : it->second;
     }
@@ -176,22 +177,6 @@ struct Tree {
         const int d[3] = {2 * q[0] + ((k >> 1) & 1), 2 * q[1] + (k & 1), dim == 3 ? 2 * q[2] + ((k >> 2) & 1) : 0};
         return find(b[i].level + 1, d);
     }
-    // coarse relation in direction o (find_neighbors.f90): exists only on the
-    // mother's boundary in that direction
-    int nb_coarse_raw(int i, const int o[3]) const
-    {
-        if (b[i].level == 0) return -1;
-        const int *q = b[i].q;
-        int c[3] = {0, 0, 0};
-        for (int d = 0; d < dim; ++d) {
-            if (o[d] > 0 && (q[d] & 1) != 1) return -1;
-            if (o[d] < 0 && (q[d] & 1) != 0) return -1;
-            const int v = q[d] + o[d];
-            c[d] = v >= 0 ? v / 2 : -((-v + 1) / 2);
-        }
-        return find(b[i].level - 1, c);
-    }
-
     // ---- relations, cached per block set ----
     // Per block, built on its first use after the block set changed (add,
     // removal): per direction the same-level neighbour, the coarse relation,
@@ -229,23 +214,26 @@ struct Tree {
         topo();
         if (t_done[i]) return;
         const int *q = b[i].q, L = b[i].level, ns = 1 << dim, mc = maxc();
+        const bool finer = L + 1 < (int)dense.size() || !map.empty();  // may level L + 1 hold blocks?
         t_mom[i] = mother_raw(i);
-        for (int k = 0; k < ns; ++k) t_dau[(size_t)i * ns + k] = daughter_raw(i, k);
+        for (int k = 0; k < ns; ++k) t_dau[(size_t)i * ns + k] = finer ? daughter_raw(i, k) : -1;
         for (int k = 0; k < nd; ++k) {
             const int *o = dirs[k];
             const size_t e = (size_t)i * nd + k;
             const int nq[3] = {q[0] + o[0], q[1] + o[1], q[2] + o[2]};
             t_same[e] = find(L, nq);
-            t_coarse[e] = nb_coarse_raw(i, o);
-            t_cover[e] = -1;
-            if (L > 0) {
-                int cu[3] = {0, 0, 0};
-                for (int d = 0; d < dim; ++d) {
-                    const int v = q[d] + o[d];
-                    cu[d] = v >= 0 ? v / 2 : -((-v + 1) / 2);
-                }
-                t_cover[e] = find(L - 1, cu);
+            // the coarse relation in direction o (find_neighbors.f90): exists
+            // only on the mother's boundary in that direction, and is the
+            // block that covers the ghost box there
+            bool leaves = L > 0;
+            int cu[3] = {0, 0, 0};
+            for (int d = 0; d < dim; ++d) {
+                const int v = q[d] + o[d];
+                cu[d] = v >= 0 ? v / 2 : -((-v + 1) / 2);
+                if (o[d] > 0 ? (q[d] & 1) != 1 : o[d] < 0 && (q[d] & 1) != 0) leaves = false;
             }
+            t_cover[e] = L > 0 ? find(L - 1, cu) : -1;
+            t_coarse[e] = leaves ? t_cover[e] : -1;
             int lo[3], hi[3];
             for (int d = 0; d < 3; ++d) {
                 if (d >= dim) lo[d] = hi[d] = 0;
@@ -262,7 +250,7 @@ struct Tree {
                     for (int cx = lo[0]; cx <= hi[0]; ++cx) {
                         const int c[3] = {2 * (q[0] + o[0]) + cx, 2 * (q[1] + o[1]) + cy,
                                           dim == 3 ? 2 * (q[2] + o[2]) + cz : 0};
-                        t_fin[e * mc + cnt++] = {find(L + 1, c), {cx, cy, cz}};
+                        t_fin[e * mc + cnt++] = {finer ? find(L + 1, c) : -1, {cx, cy, cz}};
                     }
             t_fcnt[e] = cnt;
         }
@@ -578,20 +566,30 @@ int src_sel(const Tree &T, const SyncSpec &S, int sender, bool res_pred)
     return 0;
 }
 
-// launches a cached sync: its node indices mapped to the nodes' pool slots
+// launches a cached sync: its node indices mapped to the nodes' pool slots.
+// Without filtered senders between the stages a tree that launches as it goes
+// sends all stages as one list: one upload instead of two, of the 12 syncs that
+// an adaptive 2D channel step makes.  Logged lists stay apart, so that those of
+// several trees concatenate in stage order.
 int tree_sync_run(Tree &T, const TreeSyncCache &c)
 {
-    auto patches = [&](const std::vector<wh_patch> &src) {
-        std::vector<wh_patch> out(src);
-        for (wh_patch &p : out) {
-            p.recv = T.b[p.recv].hvy;
-            p.send = T.b[p.send].hvy;
+    auto patches = [&](std::vector<wh_patch> &out, const std::vector<wh_patch> &src) {
+        for (const wh_patch &p : src) {
+            out.push_back(p);
+            out.back().recv = T.b[p.recv].hvy;
+            out.back().send = T.b[p.send].hvy;
         }
-        return out;
     };
-    if (int rc = dev_patches(T, A_U, A_T, A_FILT, patches(c.st1))) return rc;
+    const bool filtered = !c.fids[0].empty() || !c.fids[1].empty();
+    const bool together = !filtered && !T.log;
+    std::vector<wh_patch> st1, st23;
+    st1.reserve(c.st1.size() + (together ? c.st23.size() : 0));
+    patches(st1, c.st1);
+    if (together) patches(st1, c.st23);
+    if (int rc = dev_patches(T, A_U, A_T, A_FILT, std::move(st1))) return rc;
+    if (together) return WH_OK;
     // restrict_copy_at_CE's filtered senders, where the sync has any
-    if (!c.fids[0].empty() || !c.fids[1].empty()) {
+    if (filtered) {
         for (int k = 0; k < 2; ++k) {
             const int arr = k == 0 ? A_U : A_T;
             std::vector<int32_t> ids(c.fids[k]);
@@ -600,7 +598,9 @@ int tree_sync_run(Tree &T, const TreeSyncCache &c)
             if (int rc = dev_boxes(T, A_FILT, arr, boxes_of(T, c.fboxes[k]))) return rc;
         }
     }
-    return dev_patches(T, A_U, A_T, A_FILT, patches(c.st23));
+    st23.reserve(c.st23.size());
+    patches(st23, c.st23);
+    return dev_patches(T, A_U, A_T, A_FILT, std::move(st23));
 }
 
 int tree_sync(Tree &T, const SyncSpec &S)
@@ -738,6 +738,7 @@ int tree_sync(Tree &T, const SyncSpec &S)
     TreeSyncCache c;
     c.key = std::move(key);
     c.st1 = std::move(st1);
+    std::stable_sort(st23.begin(), st23.end(), [](const wh_patch &a, const wh_patch &b) { return a.stage < b.stage; });
     c.st23 = std::move(st23);
     if (filt && !restrict_senders.empty()) {
         // restrict_copy_at_CE: HD-filtered copy of every restriction sender,

@@ -775,8 +775,10 @@ static int set_patch_runs(wh_pool *P, int sync_case, const PatchRun *runs, int n
     ps.h_recv_off.push_back(npatch);
     ps.n = npatch;
     // 2D, same-level copies only: the senders of every receiver's 8
-    // directions (for the fused stages' halo gather)
-    ps.gather_ok = sync_case == 0 && P->d.dim == 2 && npatch > 0;
+    // directions (for the fused stages' halo gather).  An adaptive list has
+    // other stages; it is left before its table is cleared (nb_max rows, 0.6 MB
+    // on a pool of 16384 slots, on every step)
+    ps.gather_ok = sync_case == 0 && P->d.dim == 2 && npatch > 0 && ps.max_stage == 1;
     ps.gather_depth = -1;
     if (ps.gather_ok) {
         ps.h_gnb.assign((size_t)P->d.nb_max * 9, -1);

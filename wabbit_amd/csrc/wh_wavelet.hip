@@ -1808,15 +1808,7 @@ int run_patch_list(wh_pool *P, int array, int alt1, int alt2, const std::vector<
     }
     // validate and order by stage (lists that are already ordered are used as they are)
     const int lim[3] = {P->nx, P->ny, P->nz};
-    const auto by_stage = [](const wh_patch &a, const wh_patch &b) { return a.stage < b.stage; };
-    std::vector<wh_patch> sorted_copy;
-    const bool ordered = std::is_sorted(patches_in.begin(), patches_in.end(), by_stage);
-    if (!ordered) {
-        sorted_copy = patches_in;
-        std::stable_sort(sorted_copy.begin(), sorted_copy.end(), by_stage);
-    }
-    const std::vector<wh_patch> &p = ordered ? patches_in : sorted_copy;
-    for (const wh_patch &q : p) {
+    for (const wh_patch &q : patches_in) {
         const int op = q.op & 0xff, sel = (q.op >> 8) & 3;
         WH_CHECK(q.recv >= 0 && q.recv < P->d.nb_max && q.send >= 0 && q.send < P->d.nb_max, WH_E_ARG,
                  "patch list: hvy id out of range");
@@ -1843,6 +1835,17 @@ int run_patch_list(wh_pool *P, int array, int alt1, int alt2, const std::vector<
             }
         }
     }
+    const auto by_stage = [](const wh_patch &a, const wh_patch &b) { return a.stage < b.stage; };
+    std::vector<wh_patch> sorted_copy;
+    const bool ordered = std::is_sorted(patches_in.begin(), patches_in.end(), by_stage);
+    if (!ordered) {  // counting sort, the order within a stage kept
+        int at[5] = {0, 0, 0, 0, 0};
+        for (const wh_patch &q : patches_in) ++at[q.stage + 1];
+        for (int s = 1; s < 5; ++s) at[s] += at[s - 1];
+        sorted_copy.resize(n);
+        for (const wh_patch &q : patches_in) sorted_copy[at[q.stage]++] = q;
+    }
+    const std::vector<wh_patch> &p = ordered ? patches_in : sorted_copy;
     // 3D: the patches cut into wavefront-sized chunks (cstart[i]: patch i's first)
     std::vector<SyncChunk> chunks;
     std::vector<int> cstart(n + 1, 0);
