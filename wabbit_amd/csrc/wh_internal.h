@@ -137,12 +137,15 @@ struct WaveletWS {
     size_t patch_cap = 0;
     wh_box *d_boxes = nullptr;
     size_t box_cap = 0;
-    double *d_out = nullptr;
+    // reduction results: on the device, or in pinned space that the kernels
+    // write (out_direct: where results_reserve put the current ones)
+    double *d_out = nullptr, *h_out = nullptr;
     size_t out_cap = 0;
+    bool out_direct = false;
     // staging of the host-built lists (block ids, boxes, patches): copied to
-    // a pinned buffer and from there to the same offset of a device buffer,
-    // so that the copies run asynchronously on the pool stream; the space is
-    // reclaimed only after a stream synchronisation
+    // a pinned buffer, which kernels read where the list is short, and else
+    // from there to the same offset of a device buffer, asynchronously on the
+    // pool stream; the space is reclaimed only after a stream synchronisation
     char *h_stage = nullptr, *d_stage = nullptr;
     size_t stage_cap = 0, stage_off = 0;
     size_t pend_lo = ~(size_t)0;  // start of pieces put with defer, not yet copied
@@ -312,11 +315,12 @@ void free_wavelet_ws(wh_pool *P);
 // returns its device address; stage_sync waits for the stream and frees all
 // staged space
 int stage_begin(wh_pool *P, size_t bytes);
-// copies src into the reserved pinned space and returns the device address of
-// the same offset; the host-to-device copy is issued at once, or with defer
-// by the next stage_flush (one copy for consecutive deferred pieces of one
-// reservation)
-void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer = false);
+// copies src into the reserved pinned space and returns the address kernels
+// read it at: the pinned space itself where the list is short (longer ones with
+// once: every record has one reader), else the same offset of the device
+// buffer; that host-to-device copy is issued at once, or with defer by the next
+// stage_flush (one copy for consecutive deferred pieces of one reservation)
+void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer = false, bool once = false);
 int stage_flush(wh_pool *P);
 // copies src into the reserved pinned space and returns that host address
 // (for a direct host-to-device copy into a buffer of the caller's)
@@ -337,7 +341,7 @@ int run_detail(wh_pool *P, int array, const std::vector<int32_t> &ids, const int
 enum { WOP_FWT = 0, WOP_IWT = 1, WOP_FILTER = 2, WOP_COPY = 3, WOP_COPY_FWT = 4 };
 // per-box component maxima (|v|, SCs zeroed with zero_sc, sqrt(v*v) for
 // grouped components with sqrt_groups): out[k*neq + c]
-// Reductions launched into a caller's device range d_out (no copy, no
+// Reductions launched into a caller's range d_out of the result buffer (no copy, no
 // synchronisation), so that several of them come back in one round trip:
 // results_reserve sizes the pool's result buffer for n doubles (before any
 // of the launches), results_fetch copies them back and synchronises.

@@ -1384,6 +1384,24 @@ int filter_passes(wh_pool *P, const double *in, size_t blk_in, double *out, size
 }  // namespace
 
 static constexpr size_t STAGE_ALIGN = 256;
+// Lists that kernels read from the pinned space itself instead of a device
+// copy.  A copy costs a call on the host, a launch on the stream and a gap
+// before its reader, some 3 us each, 42 times in an adaptive 2D step; a record
+// read over the link costs its wavefront about 1 us more.
+//   once: every record has one reader (patches, chunks, boxes).  Up to 1 MB:
+//     a 2D channel of 250 blocks 1.01 -> 0.92 (64 KB) -> 0.89 (256 KB) ->
+//     0.85 ms a step (every list), 3D with 64 blocks 3.70 -> 3.62 ms; longer
+//     lists hold enough work for the copy's few us not to show.
+//   shared: id lists that each block's workgroups read again.  Up to 2 KB (512
+//     blocks; 250 blocks gain 3 %), above that the copy is as fast (4096 ids:
+//     94.2 us copied, 95.8 us read over the link).
+//   results: written once per workgroup, up to 256 KB (4096 blocks of 3
+//     components: 93 us with the copy back, 80 us without).
+static constexpr size_t STAGE_DIRECT_ONCE = (size_t)1 << 20, STAGE_DIRECT_SHARED = 2048;
+static constexpr size_t RESULTS_DIRECT = (size_t)1 << 18;
+// pinned space that kernels read and write: coherent, so that a launch sees
+// what the host wrote before it and the host what kernels wrote before a wait
+static constexpr unsigned HOST_READ = hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
 
 static size_t stage_round(size_t b) { return (b + STAGE_ALIGN - 1) / STAGE_ALIGN * STAGE_ALIGN; }
 
@@ -1414,7 +1432,7 @@ int stage_begin(wh_pool *P, size_t bytes)
     W.h_stage = W.d_stage = nullptr;
     W.stage_cap = 0;
     const size_t cap = std::max<size_t>(need, std::max<size_t>(std::max(grow, 2 * old_cap), (size_t)1 << 20));
-    WH_HIP(hipHostMalloc((void **)&W.h_stage, cap, hipHostMallocDefault));
+    WH_HIP(hipHostMalloc((void **)&W.h_stage, cap, HOST_READ));
     WH_HIP(hipMalloc((void **)&W.d_stage, cap));
     W.stage_cap = cap;
     return WH_OK;
@@ -1431,7 +1449,7 @@ int stage_flush(wh_pool *P)
     return WH_OK;
 }
 
-void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer)
+void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer, bool once)
 {
     WaveletWS &W = P->ws;
     if (!defer && stage_flush(P) != WH_OK) return nullptr;
@@ -1443,7 +1461,9 @@ void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer)
     char *h = W.h_stage + W.stage_off, *d = W.d_stage + W.stage_off;
     if (bytes) {
         std::memcpy(h, src, bytes);
-        if (defer) {
+        if (bytes <= (once ? STAGE_DIRECT_ONCE : defer ? 0 : STAGE_DIRECT_SHARED)) {
+            d = h;  // no copy: the kernel reads the pinned space
+        } else if (defer) {
             if (W.pend_lo == ~(size_t)0) W.pend_lo = W.stage_off;
         } else if (hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, P->stream) != hipSuccess) {
             set_error("staging: hipMemcpyAsync failed");
@@ -1478,6 +1498,7 @@ void free_wavelet_ws(wh_pool *P)
     if (W.d_patches) (void)hipFree(W.d_patches);
     if (W.d_boxes) (void)hipFree(W.d_boxes);
     if (W.d_out) (void)hipFree(W.d_out);
+    if (W.h_out) (void)hipHostFree(W.h_out);
     W = WaveletWS{};
 }
 
@@ -1540,7 +1561,7 @@ int run_boxes(wh_pool *P, int array, int src_array, const std::vector<wh_box> &b
                      "boxes: box outside the block");
     }
     if (int rc = stage_begin(P, sizeof(wh_box) * n)) return rc;
-    const wh_box *d_boxes = (const wh_box *)stage_put(P, boxes.data(), sizeof(wh_box) * n);
+    const wh_box *d_boxes = (const wh_box *)stage_put(P, boxes.data(), sizeof(wh_box) * n, false, true);
     if (!d_boxes) return WH_E_HIP;
     const ArrGeo A{blk_src, blk, P->cs, P->nx, P->ny, P->d.neq};
     hipLaunchKernelGGL(k_boxes, dim3(n), dim3(256), 0, P->stream, arr, src, blk_src, d_boxes, A,
@@ -1609,12 +1630,10 @@ int run_detail(wh_pool *P, int array, const std::vector<int32_t> &ids, const int
     const int n = (int)ids.size(), neq = P->d.neq;
     detail.assign((size_t)n * neq, 0.0);
     if (n == 0) return WH_OK;
-    WaveletWS &W = P->ws;
-    if (int rc = ensure(W.d_out, W.out_cap, (size_t)n * neq)) return rc;
-    if (int rc = launch_detail_list(P, array, ids, groups, W.d_out)) return rc;
-    WH_HIP(hipMemcpyAsync(detail.data(), W.d_out, sizeof(double) * n * neq, hipMemcpyDeviceToHost,
-                          P->stream));
-    if (int rc = stage_sync(P)) return rc;
+    double *d_out = nullptr;
+    if (int rc = results_reserve(P, (size_t)n * neq, &d_out)) return rc;
+    if (int rc = launch_detail_list(P, array, ids, groups, d_out)) return rc;
+    if (int rc = results_fetch(P, (size_t)n * neq, detail)) return rc;
     apply_detail_groups(detail.data(), n, detail_args(P, groups));
     return WH_OK;
 }
@@ -1636,7 +1655,7 @@ static int stage_boxes(wh_pool *P, int array, const std::vector<wh_box> &boxes, 
                      "region reduction: bad box");
     }
     if (int rc = stage_begin(P, sizeof(wh_box) * n)) return rc;
-    *d_boxes = (const wh_box *)stage_put(P, boxes.data(), sizeof(wh_box) * n);
+    *d_boxes = (const wh_box *)stage_put(P, boxes.data(), sizeof(wh_box) * n, false, true);
     return *d_boxes ? (int)WH_OK : (int)WH_E_HIP;
 }
 
@@ -1747,24 +1766,34 @@ int run_region_max(wh_pool *P, int array, const std::vector<wh_box> &boxes, bool
     const int n = (int)boxes.size(), neq = P->d.neq;
     out.assign((size_t)n * neq, 0.0);
     if (n == 0) return WH_OK;
-    WaveletWS &W = P->ws;
-    if (int rc = ensure(W.d_out, W.out_cap, (size_t)n * neq)) return rc;
-    if (int rc = launch_region_max(P, array, boxes, zero_sc, sqrt_groups, groups, W.d_out)) return rc;
-    WH_HIP(hipMemcpyAsync(out.data(), W.d_out, sizeof(double) * n * neq, hipMemcpyDeviceToHost, P->stream));
-    return stage_sync(P);
+    double *d_out = nullptr;
+    if (int rc = results_reserve(P, (size_t)n * neq, &d_out)) return rc;
+    if (int rc = launch_region_max(P, array, boxes, zero_sc, sqrt_groups, groups, d_out)) return rc;
+    return results_fetch(P, (size_t)n * neq, out);
 }
 
 int results_reserve(wh_pool *P, size_t n, double **d_out)
 {
     WaveletWS &W = P->ws;
-    if (int rc = ensure(W.d_out, W.out_cap, std::max<size_t>(n, 1))) return rc;
-    *d_out = W.d_out;
+    W.out_direct = n * sizeof(double) <= RESULTS_DIRECT;
+    if (!W.out_direct) {
+        if (int rc = ensure(W.d_out, W.out_cap, std::max<size_t>(n, 1))) return rc;
+        *d_out = W.d_out;
+        return WH_OK;
+    }
+    if (!W.h_out) WH_HIP(hipHostMalloc((void **)&W.h_out, RESULTS_DIRECT, HOST_READ));
+    *d_out = W.h_out;
     return WH_OK;
 }
 
 int results_fetch(wh_pool *P, size_t n, std::vector<double> &out)
 {
     out.assign(n, 0.0);
+    if (P->ws.out_direct) {
+        if (int rc = stage_sync(P)) return rc;
+        std::copy(P->ws.h_out, P->ws.h_out + n, out.begin());
+        return WH_OK;
+    }
     if (n) WH_HIP(hipMemcpyAsync(out.data(), P->ws.d_out, sizeof(double) * n, hipMemcpyDeviceToHost, P->stream));
     return stage_sync(P);
 }
@@ -1855,9 +1884,9 @@ int run_patch_list(wh_pool *P, int array, int alt1, int alt2, const std::vector<
             cstart[i + 1] = (int)chunks.size();
         }
     if (int rc = stage_begin(P, sizeof(wh_patch) * n + sizeof(SyncChunk) * chunks.size())) return rc;
-    const wh_patch *d_patches = (const wh_patch *)stage_put(P, p.data(), sizeof(wh_patch) * n, true);
+    const wh_patch *d_patches = (const wh_patch *)stage_put(P, p.data(), sizeof(wh_patch) * n, true, true);
     const SyncChunk *d_chunks =
-        chunks.empty() ? nullptr : (const SyncChunk *)stage_put(P, chunks.data(), sizeof(SyncChunk) * chunks.size(), true);
+        chunks.empty() ? nullptr : (const SyncChunk *)stage_put(P, chunks.data(), sizeof(SyncChunk) * chunks.size(), true, true);
     if (int rc = stage_flush(P)) return rc;
     if (!d_patches || (!chunks.empty() && !d_chunks)) return WH_E_HIP;
     int s0 = 0;
@@ -2039,9 +2068,20 @@ int wh_fwt_threshold(wh_pool *pool, int src_array, int dst_array, const int32_t 
              "wh_fwt_threshold: bad argument");
     const std::vector<int32_t> list(ids, ids + n);
     if (int rc = wh::run_blocks_op(pool, wh::WOP_FWT, src_array, dst_array, list)) return rc;
-    std::vector<double> d;
-    if (int rc = wh::run_detail(pool, dst_array, list, groups, d)) return rc;
+    // the details of the blocks whose ids the transform put on the device
     const int neq = pool->d.neq;
+    std::vector<double> d;
+    if (n > 0) {
+        WH_CHECK(neq <= 8, WH_E_ARG, "detail: at most 8 components");
+        size_t blk = 0;
+        const double *wc = wh::array_ptr(pool, dst_array, &blk, nullptr);
+        double *d_out = nullptr;
+        const wh::DetailArgs D = wh::detail_args(pool, groups);
+        if (int rc = wh::results_reserve(pool, (size_t)n * neq, &d_out)) return rc;
+        if (int rc = wh::launch_detail(pool, wc, blk, pool->ws.cur_ids, n, D, d_out)) return rc;
+        if (int rc = wh::results_fetch(pool, (size_t)n * neq, d)) return rc;
+        wh::apply_detail_groups(d.data(), n, D);
+    }
     for (int k = 0; k < n; ++k) {
         bool all = true;  // threshold_block.f90:119-124
         for (int c = 0; c < neq; ++c)
