@@ -832,18 +832,31 @@ __global__ __launch_bounds__(256) void k_copy_blocks(const double *__restrict__ 
 }
 
 // Linfty detail: per listed block and component, max over the interior of
-// |v| (sqrt(v*v) for grouped components), SC points counted as 0.
+// |v| (sqrt(v*v) for grouped components), SC points counted as 0.  Bound by
+// reading the interior rows (part of their cache lines is ghost nodes): a
+// lane requests DETAIL_Z points of a column before it compares any, and the
+// wavefronts reduce by shuffles instead of 256 atomics on one LDS word (512
+// blocks of 24^3, 4 components: 159 -> 126 us).
 struct DetailArgs {
     int g, bs[3], dim, neq;
     int groups[8];
 };
+// the maximum over a wavefront's lanes (exact in any order)
+__device__ inline double wave_max(double m)
+{
+    for (int o = 32; o > 0; o >>= 1) {
+        const double t = __shfl_xor(m, o, 64);
+        m = t > m ? t : m;
+    }
+    return m;
+}
+
+constexpr int DETAIL_Z = 8;  // a column's points requested together
 __global__ __launch_bounds__(256) void k_detail(const double *__restrict__ arr,
                                                 const int32_t *__restrict__ ids, ArrGeo A,
                                                 DetailArgs D, double *__restrict__ out)
 {
-    __shared__ unsigned long long smax;
-    if (threadIdx.x == 0) smax = 0ull;
-    __syncthreads();
+    __shared__ double wmax[4];
     const int k = (int)blockIdx.x / D.neq, c = (int)blockIdx.x - k * D.neq;
     const int b = ids[k];
     const int ncol = D.bs[0] * D.bs[1], nz = D.bs[2];
@@ -856,17 +869,28 @@ __global__ __launch_bounds__(256) void k_detail(const double *__restrict__ arr,
         const bool sc2 = ((ix & 1) == 0) && ((iy & 1) == 0);
         const double *col = u + (size_t)(zoff * A.ny + D.g + iy) * A.nx + (D.g + ix);
         const size_t zs = (size_t)A.nx * A.ny;
-        for (int iz = 0; iz < nz; ++iz) {
-            const bool sc = sc2 && (D.dim == 2 || (iz & 1) == 0);
-            const double v = sc ? 0.0 : col[iz * zs];
-            const double a = sq ? sqrt(v * v) : fabs(v);
-            m = a > m ? a : m;
+        for (int z0 = 0; z0 < nz; z0 += DETAIL_Z) {
+            double v[DETAIL_Z];
+#pragma unroll
+            for (int q = 0; q < DETAIL_Z; ++q) {
+                const int iz = z0 + q;
+                const bool sc = sc2 && (D.dim == 2 || (iz & 1) == 0);
+                v[q] = iz < nz && !sc ? col[iz * zs] : 0.0;
+            }
+#pragma unroll
+            for (int q = 0; q < DETAIL_Z; ++q) {
+                const double a = sq ? sqrt(v[q] * v[q]) : fabs(v[q]);
+                m = a > m ? a : m;
+            }
         }
     }
-    // non-negative doubles order like their bit patterns
-    atomicMax(&smax, (unsigned long long)__double_as_longlong(m));
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) out[blockIdx.x] = __longlong_as_double((long long)smax);
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w) m = wmax[w] > m ? wmax[w] : m;
+        out[blockIdx.x] = m;
+    }
 }
 
 // k_detail with one wavefront per (block, component), four per workgroup:
@@ -897,10 +921,7 @@ __global__ __launch_bounds__(256) void k_detail_wave(const double *__restrict__ 
             m = a > m ? a : m;
         }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        const double t = __shfl_xor(m, o, 64);
-        m = t > m ? t : m;
-    }
+    m = wave_max(m);
     if (lane == 0) out[item] = m;
 }
 
@@ -1009,10 +1030,12 @@ __global__ __launch_bounds__(256) void k_region_sum(const double *__restrict__ a
     }
 }
 
-// Per-box maxima (one workgroup per box): per component the max over the box
+// Per-box maxima: per component the max over the box
 // of |v| (zero_sc: SC points count as 0; sqrt_groups: components of group
 // >= 2 take sqrt(v*v)), as threshold_block with `indices` and the Linfty
-// norm of componentWiseNorm_tree.
+// norm of componentWiseNorm_tree.  A workgroup per box and component, so that
+// a few hundred boxes fill the chip (250 boxes of 24^2, 3 components: 14.2 us
+// with a workgroup per box and its components in turn, 5.6 us).
 struct RegionArgs {
     int g, dim, neq, zero_sc, sqrt_groups;
     int groups[8];
@@ -1020,28 +1043,29 @@ struct RegionArgs {
 __global__ __launch_bounds__(256) void k_region_max(const double *__restrict__ arr, const wh_box *__restrict__ boxes,
                                                     ArrGeo A, RegionArgs R, double *__restrict__ out)
 {
-    __shared__ unsigned long long smax[8];
-    if (threadIdx.x < 8) smax[threadIdx.x] = 0ull;
-    __syncthreads();
-    const wh_box B = boxes[blockIdx.x];
+    __shared__ double wmax[4];
+    const int k = (int)blockIdx.x / R.neq, c = (int)blockIdx.x - k * R.neq;
+    const wh_box B = boxes[k];
     const int n0 = B.hi[0] - B.lo[0] + 1, n1 = B.hi[1] - B.lo[1] + 1, n2 = B.hi[2] - B.lo[2] + 1;
     const int npts = n0 * n1 * n2;
-    for (int c = 0; c < R.neq; ++c) {
-        double m = 0.0;
-        const double *u = arr + (size_t)B.hvy * A.blk_in + c * A.cs;
-        for (int e = threadIdx.x; e < npts; e += blockDim.x) {
-            const int ix = B.lo[0] + e % n0, iy = B.lo[1] + (e / n0) % n1, iz = B.lo[2] + e / (n0 * n1);
-            const bool sc = (((ix - R.g) & 1) == 0) && (((iy - R.g) & 1) == 0) &&
-                            (R.dim == 2 || ((iz - R.g) & 1) == 0);
-            const double v = (R.zero_sc && sc) ? 0.0 : u[((size_t)iz * A.ny + iy) * A.nx + ix];
-            const double a = (R.sqrt_groups && R.groups[c] >= 2) ? sqrt(v * v) : fabs(v);
-            m = a > m ? a : m;
-        }
-        atomicMax(&smax[c], (unsigned long long)__double_as_longlong(m));
+    const bool sq = R.sqrt_groups && R.groups[c] >= 2;
+    const double *u = arr + (size_t)B.hvy * A.blk_in + c * A.cs;
+    double m = 0.0;
+    for (int e = threadIdx.x; e < npts; e += blockDim.x) {
+        const int ix = B.lo[0] + e % n0, iy = B.lo[1] + (e / n0) % n1, iz = B.lo[2] + e / (n0 * n1);
+        const bool sc = (((ix - R.g) & 1) == 0) && (((iy - R.g) & 1) == 0) &&
+                        (R.dim == 2 || ((iz - R.g) & 1) == 0);
+        const double v = (R.zero_sc && sc) ? 0.0 : u[((size_t)iz * A.ny + iy) * A.nx + ix];
+        const double a = sq ? sqrt(v * v) : fabs(v);
+        m = a > m ? a : m;
     }
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x < R.neq)
-        out[(size_t)blockIdx.x * R.neq + threadIdx.x] = __longlong_as_double((long long)smax[threadIdx.x]);
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w) m = wmax[w] > m ? wmax[w] : m;
+        out[blockIdx.x] = m;
+    }
 }
 
 // Coarse-extension boxes: one workgroup per box.
@@ -1755,7 +1779,7 @@ int launch_region_max(wh_pool *P, int array, const std::vector<wh_box> &boxes, b
     R.sqrt_groups = sqrt_groups;
     for (int c = 0; c < 8; ++c) R.groups[c] = (groups && c < neq) ? groups[c] : 1;
     const ArrGeo A{blk, blk, P->cs, P->nx, P->ny, neq};
-    hipLaunchKernelGGL(k_region_max, dim3(n), dim3(256), 0, P->stream, arr, d_boxes, A, R, d_out);
+    hipLaunchKernelGGL(k_region_max, dim3((unsigned)(n * neq)), dim3(256), 0, P->stream, arr, d_boxes, A, R, d_out);
     WH_HIP(hipGetLastError());
     return WH_OK;
 }
