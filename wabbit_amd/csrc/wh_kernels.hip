@@ -1748,8 +1748,11 @@ __device__ void dt_combine(double *scal, double v, const TimeDev &tc)
         __hip_atomic_fetch_min(acc, (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
     if (__hip_atomic_fetch_add(cnt, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT) + 1 != gridDim.x) return;
+    // the others' minima were released through the counter: only the last
+    // workgroup, which reads them, has to acquire
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     const double m = __longlong_as_double(
-        (long long)__hip_atomic_exchange(acc, (unsigned long long)__double_as_longlong(DT_NONE), __ATOMIC_ACQ_REL,
+        (long long)__hip_atomic_exchange(acc, (unsigned long long)__double_as_longlong(DT_NONE), __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT));
     __hip_atomic_store(cnt, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     scal[DS_DTMIN_BITS] = m;
