@@ -179,7 +179,10 @@ int wh_time_fetched(wh_pool *pool, double *time, int *iteration, double *dt_last
  * fused stage kernels (path 2 of wh_rk_step).  use_graph = 1 captures one
  * step into a hipGraph once and replays it (re-captured when the active list,
  * the patch tables or the parameters change).  Steps at or beyond time_max
- * take dt = 0 and leave the state and iteration unchanged. */
+ * take dt = 0 and leave the state and iteration unchanged.  A step whose
+ * blocks the stages refuse (WH_E_ARG) leaves time and iteration as they were;
+ * after WH_E_HIP they are undefined until wh_time_set (a step's time advance is
+ * queued before its stages). */
 int wh_run_steps(wh_pool *pool, const wh_acm_params *p, const double *butcher, int nrows,
                  const wh_time_params *tp, int nsteps, int use_graph);
 

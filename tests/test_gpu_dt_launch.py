@@ -58,3 +58,25 @@ def test_dt_between_replayed_steps():
     p.run_steps(acm, butcher_rk4(), L.time_params_c(TimeParams(time_max=time)), 1, use_graph=False)
     assert p.time_get() == (time, it, 0.0)
     p.close()
+
+
+@pytest.mark.parametrize("use_graph", [False, True])
+def test_refused_step_leaves_the_time(use_graph):
+    """A block whose tile the 2D stages refuse: time, iteration and state stay,
+    and the pool's next step starts from them."""
+    bs, g = 96, 2
+    f = EquidistantForest(2, 1, [bs, bs], g, [1.0, 1.0])
+    acm = L.acm_params_c(ACMParams(dim=2, scheme=4, penalization=False, c_0=20.0, nu=1e-3, CFL=0.5))
+    p = L.Pool(2, [bs, bs], g, 3, f.n, n_work_slots=3)
+    u = 0.2 * np.random.default_rng(1).standard_normal((f.n,) + p.block_shape())
+    p.upload(L.WH_BLOCK, 0, u)
+    p.set_active(f.active, f.x0dx)
+    p.set_patches(0, f.same_level_patches(2))
+    p.time_set(0.5, 7)
+    with pytest.raises(L.WabbitHipError) as ei:
+        p.run_steps(acm, butcher_rk4(), L.time_params_c(TimeParams(time_max=1e9)), 2, use_graph=use_graph)
+    assert ei.value.code == L.WH_E_ARG
+    assert p.time_get() == (0.5, 7, 0.0)
+    got = p.download(L.WH_BLOCK, 0, f.n)[:, :, 0, g:g + bs, g:g + bs]
+    assert np.array_equal(got, u[:, :, 0, g:g + bs, g:g + bs])
+    p.close()

@@ -1072,9 +1072,13 @@ int wh_time_fetched(wh_pool *P, double *time, int *iteration, double *dt_last)
     return WH_OK;
 }
 
+// The dt launch also advances the time: what the stages refuse is refused
+// before it.
 static int one_device_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
                            const TimeDev &tc)
 {
+    WH_CHECK(P->d.dim == 3 || P->nact == 0 || tile2d_ok(P->d.bs[0], P->d.bs[1], reach_of(a.scheme)), WH_E_ARG,
+             "2D block tile exceeds LDS");
     if (int rc = launch_dt(P, a, &tc)) return rc;
     return fused_step(P, a, bt, nrows);
 }
