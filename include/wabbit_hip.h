@@ -150,7 +150,10 @@ int wh_rk_combine(wh_pool *pool, int out_array, int base_array, int nterms,
  * block in one launch); 1: one launch per block ("plain", as the reference
  * loops over blocks); 2: fused stage kernels (RHS + RK update in one launch
  * per stage, needs a tableau whose stage rows have only a sub-diagonal
- * entry, e.g. classic RK4).  butcher is (nrows x nrows) row-major. */
+ * entry, e.g. classic RK4).  butcher is (nrows x nrows) row-major.
+ * Path 2 leaves work slots 0-2 as scratch: slot 0 holds block interiors only,
+ * packed, and so do slots 1 and 2 in a 3D pool where every face is gathered
+ * (WH_TUNE_GATHER); nothing should be read from them in the block layout. */
 int wh_rk_step(wh_pool *pool, const wh_acm_params *p, const double *butcher, int nrows,
                double time, double dt, int path);
 
@@ -176,7 +179,8 @@ int wh_time_fetched(wh_pool *pool, double *time, int *iteration, double *dt_last
 
 /* `nsteps` main-loop time steps with dt, its clamps and the time advance kept
  * on the device: per step the block-dt reduction, the clamps, a sync and the
- * fused stage kernels (path 2 of wh_rk_step).  use_graph = 1 captures one
+ * fused stage kernels (path 2 of wh_rk_step, which leaves the work slots as
+ * scratch).  use_graph = 1 captures one
  * step into a hipGraph once and replays it (re-captured when the active list,
  * the patch tables or the parameters change).  Steps at or beyond time_max
  * take dt = 0 and leave the state and iteration unchanged.  A step whose
@@ -540,7 +544,9 @@ int wh_set_tables_from_forests(wh_pool *pool, wh_forest *const *forests, int n, 
  * z-marching kernel the state's ghost nodes are filled as always, and the
  * later stages read every face that is one whole same-level copy from the
  * neighbour's interior, so that only the remaining patches are launched on
- * the stage inputs in the work slots.  0 fills the ghost nodes first. */
+ * the stage inputs in the work slots; where every face is one, the stage
+ * inputs hold block interiors only, packed as [block][dim+1][Bs2][Bs1][Bs0].
+ * 0 fills the ghost nodes first, of stage inputs in the block layout. */
 enum {
     WH_TUNE_K3D_YSPLIT = 1,
     WH_TUNE_K2D_STAGE = 2,

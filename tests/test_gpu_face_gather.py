@@ -83,3 +83,32 @@ def test_face_gather_matches_ghost_fill(bs, g, depth, scheme, skew, refined, tab
     print(bs, scheme, table, "max |diff|", np.abs(on - off).max(), flush=True)
     assert np.array_equal(on, off)
     assert np.all(np.isfinite(on))
+
+
+@pytest.mark.parametrize("refined", [0, 5])
+def test_steps_after_a_packed_step(refined):
+    """The work slots are scratch after a fused step, packed on a uniform grid:
+    the other paths, other stencils and a plain right-hand side on the same pool
+    give what they give after a step that filled every ghost node."""
+    bs, g, out = [12, 12, 12], 5, {}
+    for gather in (1, 0):
+        f = _forest(bs, g, refined)
+        _, _, hv, x = f.blocks()
+        p = L.Pool(3, bs, g, 4, 320, n_work_slots=5)
+        p.set_tuning(L.WH_TUNE_GATHER, gather)
+        p.upload(L.WH_BLOCK, 0, 0.1 * np.random.default_rng(5).standard_normal((320,) + p.block_shape()))
+        p.set_active(hv, x)
+        p.set_patches(0, f.patches(3, 3, 4))
+        got = []
+        for scheme, path in ((4, 2), (4, 0), (6, 2), (4, 2), (2, 1)):
+            ac = L.acm_params_c(ACMParams(dim=3, scheme=scheme, penalization=False, c_0=10.0, nu=1e-3))
+            p.rk_step(ac, butcher_rk4(), 0.0, 1e-4, path)
+            got.append(p.download(L.WH_BLOCK, 0, 320))
+        p.sync(L.WH_BLOCK, 0)
+        p.rhs(ac, 0.0, L.WH_BLOCK, 1)
+        got.append(p.download(L.WH_WORK + 1, 0, 320)[hv][:, :, g:-g, g:-g, g:-g])
+        out[gather] = got
+        p.close()
+        f.close()
+    for on, off in zip(out[1], out[0]):
+        assert np.array_equal(on, off) and np.all(np.isfinite(on))
