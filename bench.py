@@ -241,7 +241,6 @@ def run_adaptive(args, w):
         roofline["tuned_variant"] = s.tuned[0]
         if w["dim"] == 3:
             roofline["tuned_zsplit"] = s.pool.get_tuning(L.WH_TUNE_K3D_ZSPLIT)
-            roofline["tuned_waves"] = s.pool.get_tuning(L.WH_TUNE_K3D_WAVES)
             roofline["tuned_xcd"] = s.pool.get_tuning(L.WH_TUNE_K3D_XCD)
     cpu = None
     if not args.no_cpu:
@@ -587,7 +586,6 @@ def main():
         roofline["halo_gather"] = pool.get_tuning(L.WH_TUNE_GATHER)
     if dim == 3:
         roofline["tuned_zsplit"] = pool.get_tuning(L.WH_TUNE_K3D_ZSPLIT)
-        roofline["tuned_waves"] = pool.get_tuning(L.WH_TUNE_K3D_WAVES)
         roofline["tuned_xcd"] = pool.get_tuning(L.WH_TUNE_K3D_XCD)
 
     paths = {"fused_graph": round(value, 1)}

@@ -561,10 +561,9 @@ int wh_get_tuning(wh_pool *pool, int key, int *value);
 /* Autotuner: times every valid variant of the RHS/stage kernel for this
  * pool's (Bs, g, neq) and parameters on the current active blocks, keeps the
  * fastest and returns it (3D: the WH_TUNE_K3D_YSPLIT value, with the
- * WH_TUNE_K3D_ZSPLIT, WH_TUNE_K3D_WAVES and WH_TUNE_K3D_XCD values set as
- * well, each variant timed with the ghost fill of a stage input that it
- * needs; 2D: the
- * WH_TUNE_K2D_STAGE value).  With three or more work slots the timed kernel
+ * WH_TUNE_K3D_ZSPLIT and WH_TUNE_K3D_XCD values set as well, each variant
+ * timed with the ghost fill of a stage input that it needs; 2D, one kernel:
+ * the WH_TUNE_K2D_STAGE value as it is).  With three or more work slots the timed kernel
  * is the fused RK stage kernel and work slots 0 and 1 are overwritten,
  * otherwise the RHS kernel and work slot 1. */
 int wh_autotune(wh_pool *pool, const wh_acm_params *p, int reps, int *best_value, double *best_ms);

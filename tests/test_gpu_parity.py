@@ -16,7 +16,7 @@ from helpers import (interior, oracle_run, random_mask, rel_l2, reorder_to_fores
                      tg3d_case, vortex2d_case)
 from wabbit_amd import lib as L
 from wabbit_amd.forest import EquidistantForest
-from wabbit_amd.params import ACMParams, TimeParams
+from wabbit_amd.params import ACMParams, TimeParams, butcher_rk4
 from wabbit_amd.timestep import PATH_FUSED, PATH_PER_BLOCK, PATH_REFERENCE, AcmSolver
 
 pytestmark = pytest.mark.gpu
@@ -222,14 +222,41 @@ def test_divergence_guard_and_errors():
     pool.close()
 
 
+def _oracle_step(forest, acm, hvy, mask, dt):
+    """The interiors after one RK4 step of the oracle."""
+    po = _oracle()
+    run = po.EquidistantRun(po.make_params(acm), forest.bs[:forest.dim], forest.g, REACH[acm.scheme], acm.neq, forest.level,
+                            forest.domain[:forest.dim], hvy.copy(), forest.block_at(), mask)
+    run.step(dt)
+    return interior(run.hvy, forest.bs[0], forest.g, forest.dim)
+
+
+def _pool_step(forest, acm, hvy, mask, dt, path, tuning):
+    """The same step by a pool with these tuning values."""
+    pool = L.Pool(forest.dim, forest.bs, forest.g, acm.neq, forest.n, n_work_slots=5, n_mask=6)
+    for key, value in tuning:
+        pool.set_tuning(key, value)
+        assert pool.get_tuning(key) == value
+    pool.set_active(forest.active, forest.x0dx)
+    pool.set_patches(0, forest.same_level_patches(REACH[acm.scheme]))
+    pool.upload(L.WH_BLOCK, 0, hvy)
+    pool.upload(L.WH_MASK, 0, mask)
+    pool.rk_step(L.acm_params_c(acm), butcher_rk4(), 0.0, dt, path)
+    got = interior(pool.download(L.WH_BLOCK, 0, forest.n), forest.bs[0], forest.g, forest.dim)
+    pool.close()
+    return got
+
+
+SPLITS_3D = [(0, 1, 0), (0, 1, 1), (1, 1, 0), (2, 1, 0), (3, 1, 0), (2, 2, 0), (3, 4, 0), (2, 3, 0)]
+
+
 @pytest.mark.parametrize("scheme", [4, 6])
-@pytest.mark.parametrize("ysplit,zsplit,waves,xcd", [(0, 1, 1, 0), (0, 1, 1, 1), (0, 1, 4, 1), (1, 1, 1, 0), (2, 1, 1, 0),
-                                                     (3, 1, 1, 0), (2, 2, 1, 0), (3, 4, 1, 0), (2, 3, 3, 0),
-                                                     (3, 1, 3, 0)])
-def test_3d_kernel_variants_identical(scheme, ysplit, zsplit, waves, xcd):
-    """Every tuning variant of the 3D stage kernel (y-split, z-split, waves
-    per SIMD, XCD swizzle of the flat kernel) gives the oracle's RHS bit for
-    bit (the autotuner may pick any of them)."""
+@pytest.mark.parametrize("ysplit,zsplit,xcd", SPLITS_3D)
+def test_3d_kernel_variants_identical(scheme, ysplit, zsplit, xcd):
+    """The flat 3D stage kernel with and without its XCD swizzle and the
+    z-marching one over y-splits and z-splits (those that do not divide the
+    block fall back to others) give the oracle's RHS bit for bit; the autotuner
+    may pick any of them."""
     po = _oracle()
     forest, acm, hvy, mask = _setup(3, scheme, True, True, True, J=1, bs=24)
     hs = _oracle_sync(forest, acm, hvy, REACH[scheme])
@@ -239,9 +266,8 @@ def test_3d_kernel_variants_identical(scheme, ysplit, zsplit, waves, xcd):
     pool.upload(L.WH_MASK, 0, mask)
     pool.set_tuning(L.WH_TUNE_K3D_YSPLIT, ysplit)
     pool.set_tuning(L.WH_TUNE_K3D_ZSPLIT, zsplit)
-    pool.set_tuning(L.WH_TUNE_K3D_WAVES, waves)
     pool.set_tuning(L.WH_TUNE_K3D_XCD, xcd)
-    assert pool.get_tuning(L.WH_TUNE_K3D_ZSPLIT) == zsplit and pool.get_tuning(L.WH_TUNE_K3D_WAVES) == waves
+    assert pool.get_tuning(L.WH_TUNE_K3D_ZSPLIT) == zsplit
     pool.rhs(L.acm_params_c(acm), 0.0, L.WH_BLOCK, 1)
     got = interior(pool.download(L.WH_WORK + 1, 0, forest.n), 24, forest.g, 3)
     p = po.make_params(acm)
@@ -255,21 +281,30 @@ def test_3d_kernel_variants_identical(scheme, ysplit, zsplit, waves, xcd):
     pool.close()
 
 
+@pytest.mark.parametrize("scheme,skew", [(4, False), (6, True)])
+def test_3d_fused_step_choices_identical(scheme, skew):
+    """One fused RK4 step, penalised + sponge, by every split of the stage kernel
+    and by the automatic one, with faces gathered from the neighbours and with
+    every ghost node filled: the oracle's state bit for bit."""
+    forest, acm, hvy, mask = _setup(3, scheme, skew, True, True, J=1, bs=24)
+    want = _oracle_step(forest, acm, hvy, mask, 1e-4)
+    for ysplit, zsplit, xcd in [(-1, 1, 0)] + SPLITS_3D:
+        for gather in (1, 0):
+            got = _pool_step(forest, acm, hvy, mask, 1e-4, PATH_FUSED,
+                             [(L.WH_TUNE_K3D_YSPLIT, ysplit), (L.WH_TUNE_K3D_ZSPLIT, zsplit),
+                              (L.WH_TUNE_K3D_XCD, xcd), (L.WH_TUNE_GATHER, gather)])
+            assert np.array_equal(got, want), (ysplit, zsplit, xcd, gather)
+
+
 @pytest.mark.parametrize("scheme", SCHEMES)
 @pytest.mark.parametrize("path", [PATH_FUSED, PATH_REFERENCE])
 def test_2d_kernel_variants_identical(scheme, path):
-    """Every 2D stage-kernel variant (WH_TUNE_K2D_STAGE 0..4: plain, early
-    loads, persistent pipelined with 2/4/8 workgroups per CU) gives the same
-    state bit for bit, penalised + sponge, one RK4 step."""
+    """One RK4 step, penalised + sponge, with halos gathered from the neighbours
+    and with every ghost node filled: the oracle's state bit for bit.  The
+    values of the keys that select nothing are taken and change nothing."""
     forest, acm, hvy, mask = _setup(2, scheme, False, True, True)
-    out = {}
-    for stage in (0, 1, 2, 3, 4):
-        solver = AcmSolver(forest, acm, TimeParams(time_max=10.0), REACH[scheme], path=path, mask=mask,
-                           n_mask=6)
-        L.check(L.load().wh_set_tuning(solver.pool.h, L.WH_TUNE_K2D_STAGE, stage))
-        solver.load(hvy)
-        solver.step()
-        out[stage] = solver.state()
-        solver.pool.close()
-    for stage in (1, 2, 3, 4):
-        assert np.array_equal(out[0], out[stage]), stage
+    want = _oracle_step(forest, acm, hvy, mask, 1e-4)
+    for gather, stage, waves in ((1, 1, 1), (0, 1, 1), (1, 4, 3)):
+        got = _pool_step(forest, acm, hvy, mask, 1e-4, path,
+                         [(L.WH_TUNE_GATHER, gather), (L.WH_TUNE_K2D_STAGE, stage), (L.WH_TUNE_K3D_WAVES, waves)])
+        assert np.array_equal(got, want), (gather, stage, waves)

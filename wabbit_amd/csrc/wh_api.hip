@@ -1177,7 +1177,6 @@ int wh_set_tuning(wh_pool *P, int key, int value)
     if (key == WH_TUNE_K3D_WAVES) {
         WH_CHECK(value == 1 || value == 3 || value == 4, WH_E_ARG, "K3D_WAVES is 1, 3 or 4");
         P->k3d_waves = value;
-        P->topo_version++;
         return WH_OK;
     }
     if (key == WH_TUNE_K3D_ZSPLIT) {
@@ -1191,7 +1190,6 @@ int wh_set_tuning(wh_pool *P, int key, int value)
     if (key == WH_TUNE_K2D_STAGE) {
         WH_CHECK(value >= 0 && value <= 4, WH_E_ARG, "K2D_STAGE is 0..4");
         P->k2d_stage = value;
-        P->topo_version++;
         return WH_OK;
     }
     WH_CHECK(value >= -1 && value <= 64, WH_E_ARG, "ysplit out of range");
@@ -1272,18 +1270,18 @@ int wh_autotune(wh_pool *P, const wh_acm_params *p, int reps, int *best_value, d
     // one kernel.  The variant value is reported in best_value (3D: the
     // y-split; the z-split is set too).
     struct Var {
-        int v, zs, waves, xcd;
+        int v, zs, xcd;
     };
     std::vector<Var> cand;
     const bool three = P->d.dim == 3;
     if (three) {
-        for (int xcd : {0, 1}) cand.push_back({0, 1, 1, xcd});
+        for (int xcd : {0, 1}) cand.push_back({0, 1, xcd});
         for (int ys = 1; ys <= 8; ++ys)
             for (int zs = 1; zs <= 8; ++zs)
                 if (zm_valid(P->d.bs[0], P->d.bs[1], p->scheme, ys) && zm_zvalid(P->d.bs[2], p->scheme, zs))
-                    cand.push_back({ys, zs, 1, 0});
+                    cand.push_back({ys, zs, 0});
     } else {
-        cand.push_back({P->k2d_stage, 1, 1, 0});
+        cand.push_back({P->k2d_stage, 1, 0});
     }
     int &knob = three ? P->k3d_ysplit : P->k2d_stage;
     const AcmDev a = make_acm_dev(p);
@@ -1309,14 +1307,13 @@ int wh_autotune(wh_pool *P, const wh_acm_params *p, int reps, int *best_value, d
                                       compact, compact);
         return launch_rhs(P, a, P->block, out, P->d_active, P->d_x0dx, P->nact);
     };
-    const Var saved{knob, P->k3d_zsplit, P->k3d_waves, P->k3d_xcd};
+    const Var saved{knob, P->k3d_zsplit, P->k3d_xcd};
     Var best = saved;
     double bms = 1e300;
     auto set = [&](const Var &v) {
         knob = v.v;
         if (three) {
             P->k3d_zsplit = v.zs;
-            P->k3d_waves = v.waves;
             P->k3d_xcd = v.xcd;
         }
     };
