@@ -529,7 +529,7 @@ int wh_set_tables_from_forests(wh_pool *pool, wh_forest *const *forests, int n, 
  * into pieces of at least 2R planes, R the stencil reach, acts as 1; with the
  * automatic y-split 1 leaves the z-split to the library too).
  * WH_TUNE_K3D_WAVES (default 1): 1, 3 or 4, without effect (there is one
- * build of each 3D kernel, whose registers allow 3 to 5 waves per SIMD).
+ * build of each 3D kernel, whose registers allow 2 to 8 waves per SIMD).
  * WH_TUNE_K3D_XCD (default 0): 1 remaps the flat 3D kernel's workgroups so
  * that those of one block run on one XCD (one L2).
  * WH_TUNE_K2D_STAGE (default 1): 0 to 4, without effect (there is one 2D

@@ -304,8 +304,10 @@ static int sync_kept(wh_pool *P, const FaceGather &F, double *arr)
 // one step of the fused path; dt is taken from the device scalar DS_DT, or
 // per block from dtb (block groups).  With a 2D face table no ghost fill is
 // launched: every stage reads its blocks' halos from the neighbours'
-// interiors of its input array.  With a 3D face table the state gets its ghost fill as without it (its ghost nodes are the caller's); of
-// the fills of the stage inputs in the work slots only the kept patches run.
+// interiors of its input array.  With a 3D face table the state gets its ghost
+// fill as without it (its ghost nodes are the caller's: 4096 24^3 blocks 1.43 of
+// 9.6 ms a step); of the fills of the stage inputs in the work slots only the kept
+// patches run.
 static int fused_step(wh_pool *P, const AcmDev &a, const double *bt, int nrows,
                       const double *dtb = nullptr)
 {

@@ -311,16 +311,15 @@ int launch_sync_flat(wh_pool *P, double *arr, const wh_patch *d_patches, const S
 void free_wavelet_ws(wh_pool *P);
 // staging: stage_begin reserves `bytes` (aligned pieces included) for the
 // following stage_put calls, synchronising the stream and reusing the
-// buffer from its start when it is full; stage_put copies host data and
-// returns its device address; stage_sync waits for the stream and frees all
-// staged space
+// buffer from its start when it is full; stage_sync waits for the stream and
+// frees all staged space
 int stage_begin(wh_pool *P, size_t bytes);
 // copies src into the reserved pinned space and returns the address kernels
 // read it at: the pinned space itself where the list is short (longer ones with
-// once: every record has one reader), else the same offset of the device
-// buffer; that host-to-device copy is issued at once, or with defer by the next
+// few: a record has few readers), else the same offset of the device buffer;
+// that host-to-device copy is issued at once, or with defer by the next
 // stage_flush (one copy for consecutive deferred pieces of one reservation)
-void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer = false, bool once = false);
+void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer = false, bool few = false);
 int stage_flush(wh_pool *P);
 // copies src into the reserved pinned space and returns that host address
 // (for a direct host-to-device copy into a buffer of the caller's)

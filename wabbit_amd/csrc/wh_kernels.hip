@@ -835,7 +835,8 @@ bool zm_valid(int bs0, int bs1, int scheme, int ys)
     return sizeof(double) * 4 * (bs0 + 2 * R) * (ty0 + 2 * R) <= 64 * 1024;
 }
 
-// the 2D stages take blocks whose whole tile would fit a compute unit's LDS
+// the 2D stages take blocks whose whole tile would fit a compute unit's LDS (the
+// slabs need less of it; what was refused before them still is)
 bool tile2d_ok(int bs0, int bs1, int R)
 {
     return sizeof(double) * 3 * (bs0 + 2 * R) * (bs1 + 2 * R) <= 160 * 1024;
@@ -854,10 +855,12 @@ int slab_rows(int bs0, int bs1)
 }
 
 // y-split of the 3D stage kernel: the pool's tuned value, or of the valid
-// splits of at most 256 threads the one that leaves most lanes of a compute
-// unit's 12 resident wavefronts (3 per SIMD) with a column (whole wavefronts,
-// a count that divides 12), the widest slab among equals; 0 selects the flat
-// kernel.
+// splits (zm_valid: up to 512 threads) the one that gives most lanes of a
+// compute unit a column, reckoned as 12 resident wavefronts (3 per SIMD; the
+// widest stencils' registers leave 2) that hold whole workgroups only, the widest
+// slab among equals; 0 selects the flat kernel.  24x24 with FD4: 3 slabs of
+// 192 threads, 4 workgroups of 3 wavefronts, 768 lanes, against 2 slabs of 288,
+// 2 workgroups of 5, 576.
 static int zm_split(const wh_pool *P, const Geo &G, int scheme)
 {
     if (P->k3d_ysplit == 0) return 0;

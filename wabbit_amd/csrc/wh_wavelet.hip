@@ -1412,16 +1412,23 @@ static constexpr size_t STAGE_ALIGN = 256;
 // copy.  A copy costs a call on the host, a launch on the stream and a gap
 // before its reader, some 3 us each, 42 times in an adaptive 2D step; a record
 // read over the link costs its wavefront about 1 us more.
-//   once: every record has one reader (patches, chunks, boxes).  Up to 1 MB:
-//     a 2D channel of 250 blocks 1.01 -> 0.92 (64 KB) -> 0.89 (256 KB) ->
-//     0.85 ms a step (every list), 3D with 64 blocks 3.70 -> 3.62 ms; longer
-//     lists hold enough work for the copy's few us not to show.
+//   few: a record has few readers: one wavefront for a patch in 2D and a chunk,
+//     its chunks' wavefronts (a dozen on a 24^2 face) for a patch in 3D, the
+//     four wavefronts of a workgroup for a box, of a workgroup per component
+//     in k_region_max.  Up to 1 MB: a 2D channel of 250 blocks 1.01 -> 0.92
+//     (64 KB) -> 0.89 (256 KB) -> 0.85 ms a step (every list), 3D with 64 blocks
+//     3.70 -> 3.62 ms; longer lists hold enough work for the copy's few us not
+//     to show.  On the lists of 16 forests in one launch (64 solves, 34,000
+//     blocks) the link costs about what the copies did: k_boxes 9.1 -> 16.5 us
+//     and k_sync_patches 14.5 -> 16.4 us a launch against 0.41 ms of copies a
+//     step; with box lists above 64 KB copied that ensemble ran at 10.54 and
+//     10.44 M block-RK-stages/s, without at 10.66 and 10.45 M.
 //   shared: id lists that each block's workgroups read again.  Up to 2 KB (512
 //     blocks; 250 blocks gain 3 %), above that the copy is as fast (4096 ids:
 //     94.2 us copied, 95.8 us read over the link).
 //   results: written once per workgroup, up to 256 KB (4096 blocks of 3
 //     components: 93 us with the copy back, 80 us without).
-static constexpr size_t STAGE_DIRECT_ONCE = (size_t)1 << 20, STAGE_DIRECT_SHARED = 2048;
+static constexpr size_t STAGE_DIRECT_FEW = (size_t)1 << 20, STAGE_DIRECT_SHARED = 2048;
 static constexpr size_t RESULTS_DIRECT = (size_t)1 << 18;
 // pinned space that kernels read and write: coherent, so that a launch sees
 // what the host wrote before it and the host what kernels wrote before a wait
@@ -1473,7 +1480,7 @@ int stage_flush(wh_pool *P)
     return WH_OK;
 }
 
-void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer, bool once)
+void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer, bool few)
 {
     WaveletWS &W = P->ws;
     if (!defer && stage_flush(P) != WH_OK) return nullptr;
@@ -1485,7 +1492,7 @@ void *stage_put(wh_pool *P, const void *src, size_t bytes, bool defer, bool once
     char *h = W.h_stage + W.stage_off, *d = W.d_stage + W.stage_off;
     if (bytes) {
         std::memcpy(h, src, bytes);
-        if (bytes <= (once ? STAGE_DIRECT_ONCE : defer ? 0 : STAGE_DIRECT_SHARED)) {
+        if (bytes <= (few ? STAGE_DIRECT_FEW : defer ? 0 : STAGE_DIRECT_SHARED)) {
             d = h;  // no copy: the kernel reads the pinned space
         } else if (defer) {
             if (W.pend_lo == ~(size_t)0) W.pend_lo = W.stage_off;
