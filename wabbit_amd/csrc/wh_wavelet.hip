@@ -1419,10 +1419,11 @@ static constexpr size_t STAGE_ALIGN = 256;
 //     (64 KB) -> 0.89 (256 KB) -> 0.85 ms a step (every list), 3D with 64 blocks
 //     3.70 -> 3.62 ms; longer lists hold enough work for the copy's few us not
 //     to show.  On the lists of 16 forests in one launch (64 solves, 34,000
-//     blocks) the link costs about what the copies did: k_boxes 9.1 -> 16.5 us
-//     and k_sync_patches 14.5 -> 16.4 us a launch against 0.41 ms of copies a
-//     step; with box lists above 64 KB copied that ensemble ran at 10.54 and
-//     10.44 M block-RK-stages/s, without at 10.66 and 10.45 M.
+//     blocks) the link costs about what the copies did: a step's k_boxes 0.42
+//     -> 0.67 ms (9.1 -> 15.2 us a launch) and k_sync_patches 1.99 -> 2.30 ms
+//     (14.5 -> 17.5 us), its copies 0.59 -> 0.18 ms (182 -> 46 launches); with
+//     box lists above 64 KB copied that ensemble ran at 10.54 and 10.44 M
+//     block-RK-stages/s, without at 10.66 and 10.45 M.
 //   shared: id lists that each block's workgroups read again.  Up to 2 KB (512
 //     blocks; 250 blocks gain 3 %), above that the copy is as fast (4096 ids:
 //     94.2 us copied, 95.8 us read over the link).
